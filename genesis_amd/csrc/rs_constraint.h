@@ -216,6 +216,10 @@ __device__ inline int frictionloss_rows(const DModel& m, const S& st, int b, con
 // read-modify-writes do not go through global memory).
 struct RowJac {
     template <class R>
+    __device__ __forceinline__ void begin(const R& rows, int c, int D, int, int) const {
+        for (int k = 0; k < D; k++) rows.jac(c, k) = 0.f;
+    }
+    template <class R>
     __device__ __forceinline__ float& at(const R& rows, int c, int k) const {
         return rows.jac(c, k);
     }
@@ -260,7 +264,7 @@ __device__ inline void contact_row(const DModel& m, const S& st, int b, const DS
     f3 dd = (float)(2 * (i % 2) - 1) * (i < 2 ? d1 : d2);
     f3 n = dd * fr - nrm;
     int c = start + ic * 4 + i;
-    for (int k = 0; k < D; k++) jacc.at(rows, c, k) = 0.f;
+    jacc.begin(rows, c, D, la, lb);
     float jq = 0.f;
     for (int ab = 0; ab < 2; ab++) {
         float sign = ab == 0 ? -1.f : 1.f;

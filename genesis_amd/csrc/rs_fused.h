@@ -6,6 +6,7 @@
 #include "rs_collision.h"
 #include "rs_constraint.h"
 #include "rs_dyn.h"
+#include "rs_island_solver.h"
 #include "rs_wave.h"
 #include "rs_wave_dyn.h"
 #include "rs_wave_solver.h"
@@ -364,7 +365,8 @@ __device__ inline void wave_integrate(const DModel& m, const LState& loc, int la
 
 // One environment's substep on the calling wavefront (w = wavefront index in the workgroup).
 // kPath: 1 = models in the first row-tile class (at most kTileMaxDofs dofs), 4 = the second (up to kTileWideDofs),
-// 0 = the others, 2 = any (decided per call: the shared launch of several models). Returns the narrowphase's GJK/EPA
+// 5 = larger models with short constraint rows (island solver), 0 = the others, 2 = any (decided per call: the shared
+// launch of several models). Returns the narrowphase's GJK/EPA
 // work (see wave_narrowphase).
 template <bool kLds, int kPath = 2>
 __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, const FusedArgs& fa, int b, int w,
@@ -379,7 +381,8 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
     float* base = kLds ? slice : in_place ? (float*)((uint32_t*)(void*)st.qpos + (size_t)b * st.LS) : wk + fa.off_loc;
     float* tile = slice + fa.tile_off;
     const LState loc = make_local(base, fa);
-    const WorkRows R{wk + fa.off_jac, wk + fa.off_rowf, wk + fa.off_tmp, m.CMAX, m.D};
+    const bool islands = kPath == 5 || (kPath == 2 && fa.row_width > 0);
+    const WorkRows R{wk + fa.off_jac, wk + fa.off_rowf, wk + fa.off_tmp, m.CMAX, islands ? fa.row_width : m.D};
 
     if (!in_place) stage_local<true>(st, (uint32_t*)base, fa.n_local, b, lane);
     wave_sync();
@@ -409,10 +412,20 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
     }
     // ConstraintSolver.resolve
     if (!m.disable_constraint) {
-        wave_constraints(m, loc, st, b, R, lane, fa.tiled ? tile : nullptr);
-        if constexpr (kPath == 1) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile);
+        RowGroups Q;
+        if (islands) {
+            Q = row_groups(m, wk, fa);
+            island_constraints(m, loc, st, b, R, Q, lane, tile);
+        } else {
+            wave_constraints(m, loc, st, b, R, lane, fa.tiled ? tile : nullptr);
+        }
+        if constexpr (kPath == 5) {
+            if (fa.h_off >= 0) island_solve<true>(m, loc, st, b, R, Q, lane, tile, slice + fa.h_off);
+            else island_solve<false>(m, loc, st, b, R, Q, lane, tile, triangles_in_record(loc));
+        } else if constexpr (kPath == 1) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile);
         else if constexpr (kPath == 4) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile);
         else if constexpr (kPath == 0) wave_solve<0>(m, loc, st, b, R, lane, tile);
+        else if (islands) island_solve<false>(m, loc, st, b, R, Q, lane, tile, triangles_in_record(loc));
         else if (fa.tiled == kTileMaxDofs) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile);
         else if (fa.tiled == kTileWideDofs) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile);
         else wave_solve<0>(m, loc, st, b, R, lane, tile);
@@ -445,7 +458,7 @@ static __global__ void k_sched_flip(DState st) {
 // kGenericMaxThreads lanes (4 environments) per workgroup, so that a wavefront may hold all 512 registers of its SIMD
 // (the matrix-core Hessian keeps its 36 tile accumulators resident).
 template <bool kLds, int kOcc, int kPath>
-__global__ void __launch_bounds__(kPath == 0 ? kGenericMaxThreads : 512)
+__global__ void __launch_bounds__(kPath == 0 || kPath == 5 ? kGenericMaxThreads : 512)
 __attribute__((amdgpu_waves_per_eu(kOcc > 0 ? kOcc : 1, 8)))
 k_fused_wave(DModel m, DState st, FusedArgs fa) {
     extern __shared__ float lds_env[];

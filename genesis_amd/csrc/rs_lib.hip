@@ -86,10 +86,10 @@ struct rs_graph {
     hipGraphExec_t exec = nullptr;
 };
 
-static int64_t work_floats(const rs_model_header& h);
-static int64_t field_rows(const rs_model_header& h, int i);
+static int64_t work_floats(const rs_model_header& h, int row_width);
 
-static int64_t count_of(const rs_model_header& h, int kind) {
+// row_width: the island solver's row width (RS_N_WORK depends on it)
+static int64_t count_of(const rs_model_header& h, int kind, int row_width = 0) {
     switch (kind) {
         case RS_N_ONE: return 1;
         case RS_N_LINKS: return h.n_links;
@@ -109,7 +109,7 @@ static int64_t count_of(const rs_model_header& h, int kind) {
         case RS_N_CONSTRAINTS_DOFS: return (int64_t)h.len_constraints * h.n_dofs;
         case RS_N_BROAD: return h.max_collision_pairs_broad;
         case RS_N_SORT: return 2 * (int64_t)h.n_geoms;
-        case RS_N_WORK: return work_floats(h);
+        case RS_N_WORK: return work_floats(h, row_width);
         case RS_N_SCHED: return sched_rows();
         case RS_N_DOFS_PLANE: return h.n_dofs;
         case RS_N_ONE_PLANE: return 1;
@@ -118,14 +118,14 @@ static int64_t count_of(const rs_model_header& h, int kind) {
 }
 
 // rows per environment of state field i (at least 1, so that every plane is addressable even for empty models)
-static int64_t field_rows(const rs_model_header& h, int i) {
-    int64_t rows = count_of(h, k_state_fields[i].count) * k_state_fields[i].width;
+static int64_t field_rows(const rs_model_header& h, int i, int row_width = 0) {
+    int64_t rows = count_of(h, k_state_fields[i].count, row_width) * k_state_fields[i].width;
     return rows < 1 ? 1 : rows;
 }
 
 // Private-region offsets of the local fields and the env-major work layout of the fused kernel (floats, each
 // sub-array 16-byte aligned, each environment's slice 256-byte aligned).
-static void fused_layout(const rs_model_header& h, FusedArgs* fa) {
+static void fused_layout(const rs_model_header& h, FusedArgs* fa, int row_width) {
     auto up4 = [](int64_t x) { return (x + 3) / 4 * 4; };
     // local fields come first in the directory; the private region mirrors their packed planes row for row
     int64_t off = 0;
@@ -144,10 +144,18 @@ static void fused_layout(const rs_model_header& h, FusedArgs* fa) {
     fa->gjk_off = -1;
     fa->lds_wave = (int)up4((int64_t)kTileStride * tile_rows(h.n_dofs));
     fa->sched = 0;
+    fa->row_width = row_width;
+    fa->h_off = -1;
     const int64_t C = h.len_constraints > 0 ? h.len_constraints : 1, D = h.n_dofs;
     fa->off_loc = 0;
     fa->off_jac = (int)up4(off);
-    fa->off_rowf = (int)(fa->off_jac + up4(C * D));
+    // the jacobian rows: dense, or the island solver's row groups (rs_island_solver.h row_groups)
+    int64_t jac = up4(C * D);
+    if (row_width > 0) {
+        const int64_t G = row_group_max(h.n_equalities, h.n_dofs, h.max_contact_pairs);
+        jac = std::max(jac, up4(C * row_width + G * (row_width / 4 + 5 + D) + (6 * (int64_t)h.n_equalities + D) * D));
+    }
+    fa->off_rowf = (int)(fa->off_jac + jac);
     fa->off_tmp = (int)(fa->off_rowf + RW_COUNT * up4(C));
     fa->off_pc = (int)(fa->off_tmp + kTmpArrays * up4(C));
     fa->off_mc = (int)(fa->off_pc + up4((int64_t)kWave * (h.n_contacts_per_pair > 0 ? h.n_contacts_per_pair : 1) * 8));
@@ -157,21 +165,33 @@ static void fused_layout(const rs_model_header& h, FusedArgs* fa) {
     fa->work_stride = (total + 63) / 64 * 64;
 }
 
-// LDS slice of one wavefront: the private region (when it is in LDS) followed by the row tile
-static int tile_floats(const rs_model_header& h) { return (kTileStride * tile_rows(h.n_dofs) + 3) / 4 * 4; }
-// slice layout: [private region (LDS mode)][row tile][GJK/EPA polytope (models with mesh geoms)]
+// LDS slice of one wavefront: the private region (when it is in LDS) followed by the row tile (the island solver's: its
+// tile rows and four words per link)
+static int tile_floats(const rs_model_header& h, const FusedArgs& fa) {
+    if (fa.row_width > 0) return kTileStride * island_tile_rows(fa.row_width) + 4 * h.n_links;
+    return (kTileStride * tile_rows(h.n_dofs) + 3) / 4 * 4;
+}
+// slice layout: [private region (LDS mode)][row tile][GJK/EPA polytope (models with mesh geoms)][island triangles]
 static void set_lds_slice(const rs_model_header& h, FusedArgs* fa, bool use_lds, int slice_floats) {
     fa->tile_off = use_lds ? fa->loc_floats : 0;
-    fa->gjk_off = fa->gjk_words > 0 ? fa->tile_off + tile_floats(h) : -1;
+    fa->gjk_off = fa->gjk_words > 0 ? fa->tile_off + tile_floats(h, *fa) : -1;
     fa->lds_wave = slice_floats;
 }
 static int lds_slice_floats(const rs_model_header& h, const FusedArgs& fa, bool use_lds) {
-    return (use_lds ? fa.loc_floats : 0) + tile_floats(h) + fa.gjk_words;
+    return (use_lds ? fa.loc_floats : 0) + tile_floats(h, fa) + fa.gjk_words;
+}
+// the island solver's packed triangles follow in the slice when the workgroup's slices still fit with them (they are
+// in the record's nt_H otherwise): every step of its factor and triangular solves waits for one round trip to them
+static int slice_with_triangles(const rs_model* m, const FusedArgs& fa, bool use_lds, int* h_off) {
+    const int slice = lds_slice_floats(m->h, fa, use_lds), with_h = slice + tri4(m->h.n_dofs);
+    const bool in_lds = fa.row_width > 0 && (int64_t)fa.epb * with_h * 4 <= m->max_lds;
+    *h_off = in_lds ? slice : -1;
+    return in_lds ? with_h : slice;
 }
 
-static int64_t work_floats(const rs_model_header& h) {
+static int64_t work_floats(const rs_model_header& h, int row_width) {
     FusedArgs fa;
-    fused_layout(h, &fa);
+    fused_layout(h, &fa, row_width);
     return fa.work_stride;
 }
 
@@ -195,7 +215,7 @@ static void layout(const rs_model* m, int n_envs, int64_t* offs, int64_t* total)
     const int64_t rec = record_floats(m);
     int64_t off = 0, in_rec = 0;
     for (int i = 0; i < k_n_state_fields; i++) {
-        const int64_t rows = field_rows(m->h, i);
+        const int64_t rows = field_rows(m->h, i, m->fa.row_width);
         const bool local = is_local_kind(k_state_fields[i].count);
         if (local && rec > 0) {
             offs[i] = in_rec * 4;
@@ -454,14 +474,17 @@ static int fused_substep(const rs_model* m, const DState& st, hipStream_t s) {
     fa.sched = m->schedule && st.B >= sched_rows();
     if (fa.sched) hipLaunchKernelGGL(k_sched_flip, dim3(1), dim3(1), 0, s, st);
     const dim3 grid((unsigned)((st.B + epb - 1) / epb)), block((unsigned)(kWave * epb));
-    set_lds_slice(m->h, &fa, m->use_lds, lds_slice_floats(m->h, fa, m->use_lds));
+    int h_off = -1;
+    set_lds_slice(m->h, &fa, m->use_lds, slice_with_triangles(m, fa, m->use_lds, &h_off));
+    fa.h_off = h_off;
     const size_t lds = (size_t)epb * fa.lds_wave * 4;
     // one kernel variant per (private region, occupancy) for models with a row tile; models without one run the
     // generic-solver variants at the compiler's register budget (each class is instantiated in its own translation
-    // unit: rs_fused_t16.hip, rs_fused_t24.hip, rs_fused_gen.hip)
+    // unit: rs_fused_t16.hip, rs_fused_t24.hip, rs_fused_island.hip, rs_fused_gen.hip)
     const bool lds_on = m->use_lds != 0;
     if (fa.tiled == kTileMaxDofs) launch_fused_tile16(lds_on, m->occupancy, grid, block, lds, s, m->dm, st, fa);
     else if (fa.tiled == kTileWideDofs) launch_fused_tile24(lds_on, m->occupancy, grid, block, lds, s, m->dm, st, fa);
+    else if (fa.row_width > 0) launch_fused_island(lds_on, grid, block, lds, s, m->dm, st, fa);
     else launch_fused_generic(lds_on, grid, block, lds, s, m->dm, st, fa);
     HIP_OK(hipGetLastError());
     return RS_OK;
@@ -530,6 +553,30 @@ static bool has_convex_mesh(const rs_model_header& h, const char* blob) {
     return false;
 }
 
+// Entries per constraint row of the island solver: a row acts on at most two links, so it touches at most twice the dofs
+// of the longest chain of links (two for a row between joints). 0 for models that the row-tile solvers serve, with
+// more dofs than two per lane, or whose rows are longer than kRowWidthMax (a long chain: its rows are better taken as
+// dense, on the matrix cores).
+static int island_row_width(const rs_model_header& h, const char* blob) {
+    if (h.n_dofs <= kTileWideDofs || h.n_dofs > kIslandMaxDofs) return 0;
+    const int32_t *parent = nullptr, *d0 = nullptr, *d1 = nullptr;
+    for (int i = 0; i < k_n_model_arrays; i++) {
+        const int32_t* a = (const int32_t*)(blob + h.array_offset[i]);
+        if (!strcmp(k_model_arrays[i].name, "link_parent")) parent = a;
+        if (!strcmp(k_model_arrays[i].name, "link_dof_start")) d0 = a;
+        if (!strcmp(k_model_arrays[i].name, "link_dof_end")) d1 = a;
+    }
+    if (!parent || !d0 || !d1) return 0;
+    int longest = 1;
+    for (int l = 0; l < h.n_links; l++) {
+        int n = 0, steps = 0;
+        for (int k = l; k >= 0 && k < h.n_links && steps <= h.n_links; k = parent[k], steps++) n += d1[k] - d0[k];
+        longest = std::max(longest, n);
+    }
+    const int width = (std::min(2 * longest, h.n_dofs) + 3) / 4 * 4;
+    return width <= kRowWidthMax ? width : 0;
+}
+
 int rs_model_create(const rs_model_header* h, const void* blob, size_t blob_bytes, rs_model** out) {
     if (!h || !blob || !out) return fail(RS_E_INVALID, "rs_model_create: null argument");
     if (h->abi_version != RS_ABI_VERSION) return fail(RS_E_VERSION, "rs_model_create: ABI version mismatch");
@@ -584,7 +631,7 @@ int rs_model_create(const rs_model_header* h, const void* blob, size_t blob_byte
         return fail(RS_E_INVALID, "rs_model_create: integrator must be one of RS_INTEGRATOR_*");
     }
     static_assert(k_n_state_fields <= kMaxStateFields, "FusedArgs::loc_off too small");
-    fused_layout(m->h, &m->fa);
+    fused_layout(m->h, &m->fa, island_row_width(*h, (const char*)blob));
     d.work_stride = m->fa.work_stride;
     d.off_gjk = m->fa.off_gjk;
     // models with convex mesh geoms meet the GJK/EPA hand-over often (deep overlaps of hulls): their wavefronts may
@@ -596,9 +643,10 @@ int rs_model_create(const rs_model_header* h, const void* blob, size_t blob_byte
     if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, m->device) != hipSuccess) max_lds = 0;
     m->max_lds = max_lds < 65536 ? max_lds : 65536;
     if (hipDeviceGetAttribute(&m->n_cu, hipDeviceAttributeMultiprocessorCount, m->device) != hipSuccess) m->n_cu = 0;
-    // default launch shape: two environments per workgroup, private regions in LDS when they fit
-    m->fa.epb = 2;
-    m->use_lds = check_fused_config(m, m->fa, 2, 1) == RS_OK;
+    // default launch shape: two environments per workgroup (one with the island solver, whose triangles then fit in
+    // LDS), private regions in LDS when they fit
+    m->fa.epb = m->fa.row_width > 0 ? 1 : 2;
+    m->use_lds = check_fused_config(m, m->fa, m->fa.epb, 1) == RS_OK;
     g_err.clear();
     *out = m;
     return RS_OK;
@@ -619,7 +667,8 @@ int rs_fused_config_get(const rs_model* m, rs_fused_config* out) {
     if (!m || !out) return fail(RS_E_INVALID, "rs_fused_config_get: null argument");
     out->envs_per_block = m->fa.epb;
     out->use_lds = m->use_lds;
-    out->lds_bytes_per_env = lds_slice_floats(m->h, m->fa, m->use_lds) * 4;
+    int h_off;
+    out->lds_bytes_per_env = slice_with_triangles(m, m->fa, m->use_lds, &h_off) * 4;
     out->schedule = m->schedule;
     out->occupancy = m->occupancy;
     out->gjk_lds = m->fa.gjk_words > 0;
@@ -647,7 +696,7 @@ int rs_fused_config_set(rs_model* m, const rs_fused_config* c) {
 
 int rs_state_field_rows(const rs_model* m, int i, int64_t* rows) {
     if (!m || !rows || i < 0 || i >= k_n_state_fields) return fail(RS_E_INVALID, "rs_state_field_rows: bad argument");
-    *rows = field_rows(m->h, i);
+    *rows = field_rows(m->h, i, m->fa.row_width);
     return RS_OK;
 }
 

@@ -29,6 +29,8 @@ struct FusedArgs {
     int gjk_words;     // LDS floats per wavefront for the GJK/EPA polytope (0: the polytope stays in the work field)
     int gjk_off;       // offset of that polytope in the wavefront's LDS slice (-1: none)
     int tile_off;      // offset of the row tile (kTileStride x tile_rows(D) floats) in the wavefront's LDS slice
+    int row_width;     // entries per constraint row of the island solver (0: the model does not use it)
+    int h_off;         // offset of the island solver's packed triangles in the wavefront's LDS slice (-1: in nt_H)
     int sched;         // 1: map wavefronts to environments through the cost-ordered queues
     int loc_off[kMaxStateFields];  // private-region offset of each state field (local kinds only)
 };
@@ -48,6 +50,21 @@ __host__ __device__ constexpr int tile_rows(int n_dofs) {
 __host__ __device__ constexpr int tile_class(int n_dofs) {
     return n_dofs <= kTileMaxDofs ? kTileMaxDofs : n_dofs <= kTileWideDofs ? kTileWideDofs : 0;
 }
+
+// Island solver (models with 25 to 128 dofs whose rows touch at most kRowWidthMax of them): row width (a multiple of
+// 4), tile rows that stage the contact rows, words of LDS its island search needs (at most a tile), groups of rows, and
+// the words of a packed lower triangle of n rows, every row padded to a multiple of 4 so that rows are 16-byte aligned
+// (tri4(i) is also the offset of row i).
+constexpr int kIslandMaxDofs = 2 * kWave;
+constexpr int kRowWidthMax = 32;
+__host__ __device__ constexpr int island_tile_rows(int row_width) {
+    return row_width > kTileMinRows ? row_width : kTileMinRows;
+}
+static_assert(2 * kWave + 4 * kIslandMaxDofs <= kTileMinRows * kTileStride, "the island search uses the row tile");
+__host__ __device__ constexpr int row_group_max(int n_equalities, int n_dofs, int max_contacts) {
+    return (6 * n_equalities + 2 * n_dofs + max_contacts + 3) / 4 * 4;
+}
+__host__ __device__ constexpr int tri4(int n) { return 8 * (n >> 2) * ((n >> 2) + 1) + 4 * (n & 3) * ((n >> 2) + 1); }
 
 // Schedule: after its substep each environment appends itself to one of kSchedClasses queues by cost (its number of
 // constraint rows); the next substep concatenates the queues, costliest first, and wavefront w takes the w-th

@@ -7,6 +7,7 @@
 #pragma once
 #include "rs_constraint.h"
 #include "rs_wave.h"
+#include "rs_wave_dyn.h"
 
 namespace rs {
 
@@ -34,6 +35,9 @@ struct WorkRows {
 // a lane's column of the row tile as the staging buffer of the contact jacobian rows it builds
 struct TileJac {
     float* col;
+    __device__ __forceinline__ void begin(const WorkRows&, int, int D, int, int) const {
+        for (int k = 0; k < D; k++) col[k * kTileStride] = 0.f;
+    }
     __device__ __forceinline__ float& at(const WorkRows&, int, int k) const { return col[k * kTileStride]; }
     __device__ __forceinline__ void flush(const WorkRows& rows, int c, int D) const {
         for (int k = 0; k < D; k++) rows.jac(c, k) = col[k * kTileStride];
@@ -1127,18 +1131,11 @@ __device__ inline void wave_ls_eval_r(const DModel& m, const LState& loc, const 
     ls_it += N;
 }
 
-// solver.py:2427-2597 func_linesearch_batch (uniform control flow)
-template <int KD>
-__device__ inline float wave_linesearch(const DModel& m, const LState& loc, const WorkRows& R, int lane, float* tile) {
-    const int D = m.D;
-    float sn = 0.f;
-    if (KD == 0 && mfma_model(D)) {
-        sn = wave_dsum(D, lane, [&](int d) { return LF(search, d) * LF(search, d); });
-    } else {
-        for (int d = 0; d < D; d++) sn = sn + LF(search, d) * LF(search, d);
-    }
-    sn = sqrtf(sn);
-    float gtol = m.tolerance * m.ls_tolerance * sn * (m.meaninertia * (float)max(1, D));
+// solver.py:2427-2597 func_linesearch_batch (uniform control flow) along a direction of norm sn; ev.ls_init and
+// ev.ls_eval<N> give the cost, its slope and its curvature at step 0 and at N candidate steps
+template <class Ev>
+__device__ __forceinline__ float linesearch_body(const DModel& m, const LState& loc, float sn, Ev& ev) {
+    float gtol = m.tolerance * m.ls_tolerance * sn * (m.meaninertia * (float)max(1, m.D));
     LF(gtol, 0) = gtol;
     int ls_it = 0, res_code = 0;
     float res = 0.f;
@@ -1148,10 +1145,10 @@ __device__ inline float wave_linesearch(const DModel& m, const LState& loc, cons
         return 0.f;
     }
     LsP p0;
-    p0 = wave_ls_init_r<KD>(m, loc, R, lane, ls_it, tile);
+    p0 = ev.ls_init(ls_it);
     LsP p1;
     float a = p0.alpha - p0.grad / p0.hess;
-    wave_ls_eval_r<1>(m, loc, R, lane, &a, &p1, ls_it, tile);
+    ev.template ls_eval<1>(&a, &p1, ls_it);
     if (p0.cost < p1.cost) p1 = p0;
     bool done = false;
     if (fabsf(p1.grad) < gtol) {
@@ -1167,7 +1164,7 @@ __device__ inline float wave_linesearch(const DModel& m, const LState& loc, cons
             p2 = p1;
             p2update = 1;
             float an = p1.alpha - p1.grad / p1.hess;
-            wave_ls_eval_r<1>(m, loc, R, lane, &an, &p1, ls_it, tile);
+            ev.template ls_eval<1>(&an, &p1, ls_it);
             if (fabsf(p1.grad) < gtol) {
                 res = p1.alpha;
                 done = true;
@@ -1189,7 +1186,7 @@ __device__ inline float wave_linesearch(const DModel& m, const LState& loc, cons
         float al[3] = {p1.alpha - p1.grad / p1.hess, p1.alpha, (p1.alpha + p2.alpha) * 0.5f};
         while (ls_it < m.ls_iterations) {
             LsP c[3];
-            wave_ls_eval_r<3>(m, loc, R, lane, al, c, ls_it, tile);
+            ev.template ls_eval<3>(al, c, ls_it);
             float n1 = al[0], n2 = al[1];
             bool found = false;
             float ba = 0.f, bc = 0.f;
@@ -1231,6 +1228,56 @@ __device__ inline float wave_linesearch(const DModel& m, const LState& loc, cons
     LF(ls_result, 0) = res_code;
     LF(ls_it, 0) = ls_it;
     return res;
+}
+
+// the evaluator over rows staged through the row tile
+template <int KD>
+struct TileLs {
+    const DModel& m;
+    const LState& loc;
+    const WorkRows& R;
+    int lane;
+    float* tile;
+    __device__ __forceinline__ LsP ls_init(int& ls_it) { return wave_ls_init_r<KD>(m, loc, R, lane, ls_it, tile); }
+    template <int N>
+    __device__ __forceinline__ void ls_eval(const float* al, LsP* out, int& ls_it) {
+        wave_ls_eval_r<N>(m, loc, R, lane, al, out, ls_it, tile);
+    }
+};
+
+template <int KD>
+__device__ inline float wave_linesearch(const DModel& m, const LState& loc, const WorkRows& R, int lane, float* tile) {
+    const int D = m.D;
+    float sn = 0.f;
+    if (KD == 0 && mfma_model(D)) {
+        sn = wave_dsum(D, lane, [&](int d) { return LF(search, d) * LF(search, d); });
+    } else {
+        for (int d = 0; d < D; d++) sn = sn + LF(search, d) * LF(search, d);
+    }
+    sn = sqrtf(sn);
+    TileLs<KD> ev{m, loc, R, lane, tile};
+    return linesearch_body(m, loc, sn, ev);
+}
+
+// the constraint forces of the rows (ConstraintState.efc_force), from the work field to the state slab, and the
+// contacts' forces
+__device__ inline void export_row_forces(const DModel& m, const LState& loc, const DState& st, int b,
+                                         const WorkRows& R, int lane) {
+    const int n_rows = LF(n_con, 0);
+    for (int c = lane; c < n_rows; c += kWave) st.efc_force[(size_t)c * st.B + b] = R.force(c);
+    const int cs = LF(n_con_eq, 0) + LF(n_con_fl, 0);
+    const int ncont = LF(n_contacts, 0);
+    for (int i = lane; i < ncont; i += kWave) {
+        f3 nrm = ld3(st.contact_normal, i, st.B, b);
+        float fr = st.contact_friction[(size_t)i * st.B + b];
+        f3 d1, d2, f = zero3();
+        orthogonals(nrm, d1, d2);
+        for (int k = 0; k < 4; k++) {
+            f3 dd = (float)(2 * (k % 2) - 1) * (k < 2 ? d1 : d2);
+            f = f + (dd * fr - nrm) * R.force(i * 4 + k + cs);
+        }
+        st3(st.contact_force, i, st.B, b, f);
+    }
 }
 
 // solver.py:2936-3059 (init), :3063-3139 (Newton or conjugate-gradient iteration), :3164-3190 (body), :3241-3261,
@@ -1362,22 +1409,7 @@ __device__ inline void wave_solve(const DModel& m, const LState& loc, const DSta
     if (lane_dofs ? wave_ballot(nan_seen) != 0 : nan_seen) LF(errbits, 0) = LF(errbits, 0) | RS_ERR_INVALID_FORCE_NAN;
     if (lane_dofs) wave_sync();
     LF(is_warmstart, 0) = 1;
-    // the constraint forces of the rows (ConstraintState.efc_force), from the work field to the state slab
-    const int n_rows = LF(n_con, 0);
-    for (int c = lane; c < n_rows; c += kWave) st.efc_force[(size_t)c * st.B + b] = R.force(c);
-    const int cs = LF(n_con_eq, 0) + LF(n_con_fl, 0);
-    const int ncont = LF(n_contacts, 0);
-    for (int i = lane; i < ncont; i += kWave) {
-        f3 nrm = ld3(st.contact_normal, i, st.B, b);
-        float fr = st.contact_friction[(size_t)i * st.B + b];
-        f3 d1, d2, f = zero3();
-        orthogonals(nrm, d1, d2);
-        for (int k = 0; k < 4; k++) {
-            f3 dd = (float)(2 * (k % 2) - 1) * (k < 2 ? d1 : d2);
-            f = f + (dd * fr - nrm) * R.force(i * 4 + k + cs);
-        }
-        st3(st.contact_force, i, st.B, b, f);
-    }
+    export_row_forces(m, loc, st, b, R, lane);
     wave_sync();
 }
 

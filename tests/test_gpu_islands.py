@@ -1,0 +1,102 @@
+"""The fused step of models with 25 to 128 dofs and short constraint rows (rs_island_solver.h): one substep from
+identical state against the per-stage step, at the sizes and orders where the island solver's bookkeeping can go wrong:
+the smallest and the largest dof count, islands of one body, of chains and of the whole model, rows of every kind
+(connect, weld, joint equality, friction loss, contact, limit), dofs in both halves of the wavefront, and the packed
+triangles in LDS (one environment per workgroup) and in the state record (two and four)."""
+
+from __future__ import annotations
+
+import os
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from genesis_amd import scenes
+from genesis_amd.model.compiler import SolverOptions, compile_model
+from genesis_amd.model.mjcf import load_mjcf
+from genesis_amd.model.primitives import box_entity, plane_entity, sphere_entity
+from tests.parity import check_fused_matches_plain
+
+pytestmark = pytest.mark.gpu
+
+ARM = """<mujoco model="arm"><worldbody><body name="a" pos="{x} 0 0.3">
+  <joint name="j1" type="hinge" axis="0 1 0" range="-0.3 0.3" limited="true" frictionloss="0.2"/>
+  <inertial pos="0.1 0 0" mass="1" diaginertia="0.01 0.02 0.03"/>
+  <geom type="capsule" fromto="0 0 0 0.2 0 0" size="0.04"/>
+  <body name="b" pos="0.2 0 0"><joint name="j2" type="slide" axis="1 0 0" range="-0.05 0.05" limited="true"/>
+    <inertial pos="0.1 0 0" mass="0.5" diaginertia="0.01 0.02 0.03"/>
+    <geom type="sphere" size="0.06" pos="0.1 0 0"/></body></body></worldbody>
+  <equality><joint joint1="j1" joint2="j2" polycoef="0.02 0.5 0 0 0"/></equality></mujoco>"""
+
+
+def _boxes(n, spacing, opts):
+    """n free boxes with their centres ``spacing`` apart on a line, alternating with spheres."""
+    ents = [plane_entity(friction=0.5)]
+    for i in range(n):
+        pos = np.array([spacing * i, 0.01 * (i % 3), 0.049])
+        if i % 4 == 3:
+            ents.append(sphere_entity(0.05, pos, np.array([1.0, 0, 0, 0]), rho=500.0, friction=0.5, name=f"s{i}"))
+        else:
+            ents.append(box_entity(np.full(3, 0.1), pos, np.array([1.0, 0, 0, 0]), rho=500.0, friction=0.5, name=f"b{i}"))
+    return compile_model(ents, SolverOptions(dt=0.01, **opts))
+
+
+def _arms(tmp_path, n, opts):
+    ents = [plane_entity()]
+    for i in range(n):
+        p = os.path.join(str(tmp_path), f"arm{i}.xml")
+        with open(p, "w") as f:
+            f.write(ARM.format(x=0.33 * i))
+        ents.append(load_mjcf(p, f"arm{i}"))
+    return compile_model(ents, SolverOptions(dt=0.01, **opts))
+
+
+def _loops(tmp_path, n, opts):
+    return compile_model([load_mjcf(scenes.CLOSED_LOOPS_XML, f"l{i}") for i in range(n)], SolverOptions(dt=0.005, **opts))
+
+
+def _quads(tmp_path, n, opts):
+    return compile_model([plane_entity()] + [load_mjcf(scenes.QUADRUPED_XML, f"q{i}") for i in range(n)],
+                         SolverOptions(dt=0.005, **opts))
+
+
+MODELS = {
+    "boxes_apart_30": lambda t, o: _boxes(5, 0.5, o),  # islands of one body
+    "boxes_touching_30": lambda t, o: _boxes(5, 0.099, o),  # one island
+    "boxes_pairs_126": lambda t, o: _boxes(21, 0.0995, o),  # one island over both halves of the wavefront
+    "arms_26": lambda t, o: _arms(t, 13, o),  # friction, joint equality, limit and contact rows; two-dof entities
+    "arms_128": lambda t, o: _arms(t, 64, o),  # every position of a lane used
+    "loops_30": lambda t, o: _loops(t, 3, o),  # connect and weld rows
+    "quadrupeds_36": lambda t, o: _quads(t, 2, o),  # overlapping robots: long rows, 18-dof entities
+}
+
+
+@pytest.mark.parametrize("epb", [1, 2, 4])
+@pytest.mark.parametrize("name", list(MODELS))
+def test_island_step_matches_the_per_stage_step(tmp_path, name, epb):
+    from genesis_amd import runtime as rt
+
+    rt.load_library()
+    model = MODELS[name](tmp_path, {})
+    assert 24 < model.n_dofs <= 128
+    dm = rt.DeviceModel(model)
+    dm.set_fused_config(epb, False, False, 0)
+    B = 17
+    a = rt.StateSlab(dm, B)
+    gen = torch.Generator().manual_seed(5)
+    a["vel"].copy_(0.3 * torch.randn(model.n_dofs, B, generator=gen))
+    if name.startswith("arms"):
+        a["qpos"].copy_(0.4 * torch.randn(model.n_qs, B, generator=gen))
+    a.forward_kinematics()
+    a.step(3, rt.RS_MODE_PLAIN)
+    torch.cuda.synchronize()
+    b = rt.StateSlab(dm, B)
+    b.buffer.copy_(a.buffer)
+    print(f"[islands] {name} D={model.n_dofs} rows up to {int(a['n_con'].max())} config={dm.fused_config}", flush=True)
+    a.step(1, rt.RS_MODE_PLAIN)
+    b.step(1, rt.RS_MODE_FUSED)
+    torch.cuda.synchronize()
+    assert int(a["n_con"].max()) > 0
+    check_fused_matches_plain(a, b, model)
