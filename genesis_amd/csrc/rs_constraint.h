@@ -215,6 +215,7 @@ __device__ inline int frictionloss_rows(const DModel& m, const S& st, int b, con
 // copied to the row store once the row is complete (the fused kernel stages in LDS, so that the walk's
 // read-modify-writes do not go through global memory).
 struct RowJac {
+    static constexpr bool kBatch = false;
     template <class R>
     __device__ __forceinline__ void begin(const R& rows, int c, int D, int, int) const {
         for (int k = 0; k < D; k++) rows.jac(c, k) = 0.f;
@@ -247,7 +248,7 @@ struct ChainLds {
 // solver.py:580-685 add_collision_constraints, row i (0..3) of contact ic: row start + 4 ic + i (pyramid direction
 // +-d1, +-d2 from the contact normal). The impedance depends on the contact only.
 template <class R, class S, class J, class C>
-__device__ inline void contact_row(const DModel& m, const S& st, int b, const DState& cs, int cb, const R& rows,
+__device__ __forceinline__ void contact_row(const DModel& m, const S& st, int b, const DState& cs, int cb, const R& rows,
                                    int ic, int i, int start, const J& jacc, const C& chain) {
     const int D = m.D;
     const size_t CB = (size_t)cs.B;
@@ -272,6 +273,31 @@ __device__ inline void contact_row(const DModel& m, const S& st, int b, const DS
         while (link > -1) {
             f3 tpos = cpos - LD3(root_COM, link);
             const int k0 = chain.dof_start(link), k1 = chain.dof_end(link), lp = chain.parent(link);
+            if constexpr (J::kBatch) {
+                if (k1 - k0 == 6) {  // a free joint: its dofs' values are loaded together, its entries are distinct
+                    f3 ca[6], cv[6];
+                    float v[6], old[6];
+                    float* e[6];
+#pragma unroll
+                    for (int u = 0; u < 6; u++) {
+                        ca[u] = LD3(cdof_ang, k1 - 1 - u);
+                        cv[u] = LD3(cdof_vel, k1 - 1 - u);
+                        v[u] = SF(vel, k1 - 1 - u);
+                        e[u] = &jacc.at(rows, c, k1 - 1 - u);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 6; u++) old[u] = *e[u];
+#pragma unroll
+                    for (int u = 0; u < 6; u++) {
+                        const f3 vel = qrot(cv[u] - cross3(tpos, ca[u]), qident());
+                        const float jj = dot3(sign * vel, n);
+                        jq = jq + jj * v[u];
+                        *e[u] = old[u] + jj;
+                    }
+                    link = lp;
+                    continue;
+                }
+            }
             for (int k = k1 - 1; k >= k0; k--) {
                 f3 ca = LD3(cdof_ang, k), cv = LD3(cdof_vel, k);
                 f3 vel = qrot(cv - cross3(tpos, ca), qident());
@@ -293,7 +319,7 @@ __device__ inline void contact_row(const DModel& m, const S& st, int b, const DS
 }
 
 template <class R, class S, class J = RowJac>
-__device__ inline void contact_row(const DModel& m, const S& st, int b, const DState& cs, int cb, const R& rows,
+__device__ __forceinline__ void contact_row(const DModel& m, const S& st, int b, const DState& cs, int cb, const R& rows,
                                    int ic, int i, int start, const J& jacc = J()) {
     contact_row(m, st, b, cs, cb, rows, ic, i, start, jacc, ChainModel{m});
 }

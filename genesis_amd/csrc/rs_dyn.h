@@ -5,10 +5,10 @@
 
 namespace rs {
 
-// forward_kinematics.py:580-736 func_forward_kinematics_entity
+// forward_kinematics.py:580-736 func_forward_kinematics_entity, links l0 .. l1 - 1
 template <class S>
-__device__ inline void dev_forward_kinematics(const DModel& m, const S& st, int b) {
-    for (int l = 0; l < m.L; l++) {
+__device__ inline void dev_forward_kinematics(const DModel& m, const S& st, int b, int l0, int l1) {
+    for (int l = l0; l < l1; l++) {
         f3 pos = mvec3(m.link_pos, l);
         f4q quat = mquat(m.link_quat, l);
         int par = m.link_parent[l];
@@ -66,10 +66,15 @@ __device__ inline void dev_forward_kinematics(const DModel& m, const S& st, int 
     }
 }
 
-// forward_kinematics.py:337-576 func_COM_links_entity
 template <class S>
-__device__ inline void dev_com_links(const DModel& m, const S& st, int b) {
-    for (int e = 0; e < m.E; e++) {
+__device__ inline void dev_forward_kinematics(const DModel& m, const S& st, int b) {
+    dev_forward_kinematics(m, st, b, 0, m.L);
+}
+
+// forward_kinematics.py:337-576 func_COM_links_entity of entity e
+template <class S>
+__device__ inline void dev_com_links(const DModel& m, const S& st, int b, int e) {
+    {
         int l0 = m.entity_link_start[e], l1 = m.entity_link_end[e];
         // root accumulators live in root_COM (as the weighted sum) and cinr_mass (as mass_sum) until normalised
         for (int l = l0; l < l1; l++) {
@@ -143,6 +148,11 @@ __device__ inline void dev_com_links(const DModel& m, const S& st, int b) {
     }
 }
 
+template <class S>
+__device__ inline void dev_com_links(const DModel& m, const S& st, int b) {
+    for (int e = 0; e < m.E; e++) dev_com_links(m, st, b, e);
+}
+
 // forward_kinematics.py:828-864 func_update_geoms_entity
 template <class S>
 __device__ inline void dev_update_geoms(const DModel& m, const S& st, int b, bool force_fixed) {
@@ -157,10 +167,10 @@ __device__ inline void dev_update_geoms(const DModel& m, const S& st, int b, boo
     }
 }
 
-// forward_kinematics.py:993-1116 func_forward_velocity_entity
+// forward_kinematics.py:993-1116 func_forward_velocity_entity, links l0 .. l1 - 1
 template <class S>
-__device__ inline void dev_forward_velocity(const DModel& m, const S& st, int b) {
-    for (int l = 0; l < m.L; l++) {
+__device__ inline void dev_forward_velocity(const DModel& m, const S& st, int b, int l0, int l1) {
+    for (int l = l0; l < l1; l++) {
         f3 cv = zero3(), ca = zero3();
         int p = m.link_parent[l];
         if (p != -1) {
@@ -205,6 +215,11 @@ __device__ inline void dev_forward_velocity(const DModel& m, const S& st, int b)
         ST3(cd_vel, l, cv);
         ST3(cd_ang, l, ca);
     }
+}
+
+template <class S>
+__device__ inline void dev_forward_velocity(const DModel& m, const S& st, int b) {
+    dev_forward_velocity(m, st, b, 0, m.L);
 }
 
 template <class S>
@@ -419,11 +434,11 @@ __device__ inline void dev_torque_passive(const DModel& m, const S& st, int b) {
     }
 }
 
-// forward_dynamics.py:1186-1285 func_update_acc
+// forward_dynamics.py:1186-1285 func_update_acc, entities e0, e0 + step, ...
 template <class S>
-__device__ inline void dev_update_acc(const DModel& m, const S& st, int b, bool cacc) {
+__device__ inline void dev_update_acc(const DModel& m, const S& st, int b, bool cacc, int e0 = 0, int step = 1) {
     f3 g = mk3(m.gx, m.gy, m.gz);
-    for (int e = 0; e < m.E; e++) {
+    for (int e = e0; e < m.E; e += step) {
         float gc = 1.f - m.entity_gravity_compensation[e];
         for (int l = m.entity_link_start[e]; l < m.entity_link_end[e]; l++) {
             int p = m.link_parent[l];

@@ -369,8 +369,8 @@ __device__ inline void wave_integrate(const DModel& m, const LState& loc, int la
 // launch of several models). Returns the narrowphase's GJK/EPA
 // work (see wave_narrowphase).
 template <bool kLds, int kPath = 2>
-__device__ __forceinline__ int fused_env(const DModel& m, const DState& st, const FusedArgs& fa, int b, int w,
-                                          float* lds_env) {
+__device__ __forceinline__ int fused_env(const DModel& m, const DState& st, const FusedArgs& fa,
+                                          const RS_CONST int* loc_off, int b, int w, float* lds_env) {
     const int lane = lane_id();
     float* wk = st.wk + (size_t)b * fa.work_stride;
     float* slice = lds_env + (size_t)w * fa.lds_wave;
@@ -380,8 +380,8 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
     const bool in_place = !kLds && st.LS > 0;
     float* base = kLds ? slice : in_place ? (float*)((uint32_t*)(void*)st.qpos + (size_t)b * st.LS) : wk + fa.off_loc;
     float* tile = slice + fa.tile_off;
-    const LState loc = make_local(base, fa);
-    const bool islands = kPath == 5 || (kPath == 2 && fa.row_width > 0);
+    const LState loc = make_local(base, loc_off);
+    const bool islands = kPath == 5 || (kPath == 2 && fa.islands);
     const WorkRows R{wk + fa.off_jac, wk + fa.off_rowf, wk + fa.off_tmp, m.CMAX, islands ? fa.row_width : m.D};
 
     if (!in_place) stage_local<true>(st, (uint32_t*)base, fa.n_local, b, lane);
@@ -392,11 +392,12 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
     if constexpr (kPath == 1 || kPath == 4)
         if (FP(loc, n_con)[0] >= kSchedHeavyRows) __builtin_amdgcn_s_setprio(3);
     // kernel_step_1: CRBA, L^T D L, actuation + passive + bias forces, acc_smooth
-    wave_mass_matrix(m, loc, lane);
+    constexpr bool kMany = kPath != 1 && kPath != 4;
+    wave_mass_matrix<kMany>(m, loc, lane);
     wave_factor_mass(m, loc, lane);
     wave_torque_passive(m, loc, lane);
-    wave_update_acc(m, loc, lane, false);
-    wave_rne_and_qacc(m, loc, lane);
+    wave_update_acc<kMany>(m, loc, lane, false);
+    wave_rne_and_qacc<kMany>(m, loc, lane);
     // Collider.detection
     int gjk_work = 0;
     if (m.enable_collision) {
@@ -417,7 +418,8 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
             Q = row_groups(m, wk, fa);
             island_constraints(m, loc, st, b, R, Q, lane, tile);
         } else {
-            wave_constraints(m, loc, st, b, R, lane, fa.tiled ? tile : nullptr);
+            wave_constraints(m, loc, st, b, R, lane, tile, kPath == 1 || kPath == 4 || (kPath == 2 && fa.tiled != 0),
+                             fa.row_width);
         }
         if constexpr (kPath == 5) {
             if (fa.h_off >= 0) island_solve<true>(m, loc, st, b, R, Q, lane, tile, slice + fa.h_off);
@@ -431,10 +433,10 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
         else wave_solve<0>(m, loc, st, b, R, lane, tile);
     }
     // kernel_step_2: cacc, semi-implicit Euler, forward kinematics and velocities
-    wave_update_acc(m, loc, lane, true);
+    wave_update_acc<kMany>(m, loc, lane, true);
     if (m.integrator != RS_INTEGRATOR_APPROXIMATE_IMPLICITFAST) dev_implicit_damping(m, loc, 0);
     wave_integrate(m, loc, lane);
-    wave_kinematics(m, loc, lane);
+    wave_kinematics<kMany>(m, loc, lane);
     if (!in_place) stage_local<false>(st, (uint32_t*)base, fa.n_local, b, lane);
     return gjk_work;
 }
@@ -453,14 +455,26 @@ static __global__ void k_sched_flip(DState st) {
     for (int k = 0; k < kSchedClasses; k++) ctl[1 + (par ^ 1) * kSchedClasses + k] = 0;
 }
 
-// kOcc > 0 asks the compiler for at least kOcc wavefronts per SIMD (fewer registers, more spills); 0 leaves the
-// register budget to the compiler. The autotuner picks between them. Models above 24 dofs (kPath 0) run at most
-// kGenericMaxThreads lanes (4 environments) per workgroup, so that a wavefront may hold all 512 registers of its SIMD
-// (the matrix-core Hessian keeps its 36 tile accumulators resident).
-template <bool kLds, int kOcc, int kPath>
-__global__ void __launch_bounds__(kPath == 0 || kPath == 5 ? kGenericMaxThreads : 512)
-__attribute__((amdgpu_waves_per_eu(kOcc > 0 ? kOcc : 1, 8)))
-k_fused_wave(DModel m, DState st, FusedArgs fa) {
+// The arguments of a launch for larger models, which its kernels reach through the kernel-argument segment's own pointer.
+// A parameter passed by value is copied to every lane's scratch memory as soon as the compiler forms one pointer to two of
+// its members (two branches that read different members are enough) or a function that takes it by reference is not
+// inlined. Then every model array's address comes from a vector load of scratch memory instead of a scalar load, and
+// LState's offsets, cast to the constant address space from such a copy, are an address that scalar loads fault on. The
+// kernels of the smaller models take theirs by value (5% faster: the compiler may load those ahead of a branch) and must
+// keep all their functions inlined.
+struct FusedKernArgs {
+    DModel m;
+    DState st;
+    FusedArgs fa;
+};
+__device__ __forceinline__ const RS_CONST FusedKernArgs* kern_args() {
+    return (const RS_CONST FusedKernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
+// the wavefront's environment of a launch: blockIdx order, or the schedule's
+template <bool kLds, int kPath>
+__device__ __forceinline__ void fused_launch(const DModel& m, const DState& st, const FusedArgs& fa,
+                                             const RS_CONST int* loc_off) {
     extern __shared__ float lds_env[];
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     int b = xcd_block((int)blockIdx.x, (int)gridDim.x) * fa.epb + w;
@@ -486,13 +500,29 @@ k_fused_wave(DModel m, DState st, FusedArgs fa) {
         }
     }
     if (b >= st.B) return;  // whole wavefronts only
-    const int gjk_work = fused_env<kLds, kPath>(m, st, fa, b, w, lds_env);
+    const int gjk_work = fused_env<kLds, kPath>(m, st, fa, loc_off, b, w, lds_env);
     if (fa.sched && lane_id() == 0) {
         const int cls = sched_class(FV(st, n_con, b)[0], gjk_work);
         const int q = par ^ 1;
         const int slot = atomicAdd(&ctl[1 + q * kSchedClasses + cls], 1);
         if (slot < st.B) st.sched[(size_t)(q * kSchedClasses + cls) * st.B + slot] = b;
     }
+}
+
+// kOcc > 0 asks the compiler for at least kOcc wavefronts per SIMD (fewer registers, more spills); 0 leaves the
+// register budget to the compiler. The autotuner picks between them.
+template <bool kLds, int kOcc, int kPath>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kOcc > 0 ? kOcc : 1, 8)))
+k_fused_wave(DModel m, DState st, FusedArgs fa) {
+    fused_launch<kLds, kPath>(m, st, fa, (const RS_CONST int*)fa.loc_off);
+}
+
+// Models above 24 dofs (kPath 5 and 0): at most kGenericMaxThreads lanes (4 environments) per workgroup, so that a
+// wavefront may hold all 512 registers of its SIMD.
+template <bool kLds, int kPath>
+__global__ void __launch_bounds__(kGenericMaxThreads) k_fused_large(FusedKernArgs) {
+    const FusedKernArgs& a = *(const FusedKernArgs*)kern_args();
+    fused_launch<kLds, kPath>(a.m, a.st, a.fa, kern_args()->fa.loc_off);
 }
 
 // One batch of a shared launch: a model, its state slab, and the first workgroup that serves it.
@@ -510,12 +540,15 @@ __global__ void __launch_bounds__(512) k_fused_multi(const FusedSegment* __restr
     extern __shared__ float lds_env[];
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
+    // the table does not change while the kernel runs: read through the constant address space, its entries (the model's
+    // and the slab's pointers among them) are scalar loads
+    const FusedSegment* tab = (const FusedSegment*)(const RS_CONST FusedSegment*)(uintptr_t)segs;
     int s = 0;
-    while (s + 1 < n_segs && segs[s + 1].first_block <= blk) s++;
-    const FusedSegment& g = segs[s];
+    while (s + 1 < n_segs && tab[s + 1].first_block <= blk) s++;
+    const FusedSegment& g = tab[s];
     const int b = (blk - g.first_block) * g.fa.epb + w;
     if (b >= g.st.B) return;
-    fused_env<kLds>(g.m, g.st, g.fa, b, w, lds_env);
+    fused_env<kLds>(g.m, g.st, g.fa, (const RS_CONST int*)g.fa.loc_off, b, w, lds_env);
 }
 
 }  // namespace rs

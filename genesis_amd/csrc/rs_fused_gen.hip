@@ -5,8 +5,8 @@ namespace rs {
 
 void launch_fused_generic(bool use_lds, dim3 grid, dim3 block, size_t lds, hipStream_t s, const DModel& m,
                           const DState& st, const FusedArgs& fa) {
-    if (use_lds) hipLaunchKernelGGL((k_fused_wave<true, 0, 0>), grid, block, lds, s, m, st, fa);
-    else hipLaunchKernelGGL((k_fused_wave<false, 0, 0>), grid, block, lds, s, m, st, fa);
+    if (use_lds) hipLaunchKernelGGL((k_fused_large<true, 0>), grid, block, lds, s, FusedKernArgs{m, st, fa});
+    else hipLaunchKernelGGL((k_fused_large<false, 0>), grid, block, lds, s, FusedKernArgs{m, st, fa});
 }
 
 }  // namespace rs

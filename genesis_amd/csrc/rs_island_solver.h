@@ -1,5 +1,5 @@
 // Constraint rows and Newton / conjugate-gradient solve of one environment on one wavefront, for models with 25 to 128
-// dofs whose constraint rows are short (constraint/solver.py: rows :580-1286, solve :2936-3261, line search :2034-2597).
+// dofs whose constraint rows are short, except those with contacts from perturbed MPR detections (takes_islands) (constraint/solver.py: rows :580-1286, solve :2936-3261, line search :2034-2597).
 //
 // A constraint row touches the dofs above the (at most) two links it acts on: 12 of the 120 dofs of a pile of 20 free
 // boxes. So a row is kept as its W = FusedArgs::row_width first entries, the dofs' columns in ascending order (columns
@@ -14,8 +14,7 @@
 //
 // What it replaced: dense 120-column rows on the matrix cores and a rank-1 update of the dense factor for every row
 // that changed its active flag, one column after the other through memory. Pile of 20 boxes x 1024, the first four
-// steps from a reset (320 rows, 5 Newton iterations): 6.0 -> 1.32 ms per step; 101 columns of stacked boxes (380 rows):
-// 5.8 -> 1.38 ms. Of the old step's 9.4 M cycles per environment 4.3 M were the rank-1 updates, 1.0 M each the Hessian
+// steps from a reset (320 rows, 5 Newton iterations): 6.0 -> 0.94 ms per step. Of the old step's 9.4 M cycles per environment 4.3 M were the rank-1 updates, 1.0 M each the Hessian
 // and the line searches, 0.8 M the triangular solves, 0.6 M each the row builder and the updates of the row forces.
 #pragma once
 #include "rs_constraint.h"
@@ -117,41 +116,12 @@ __device__ inline void compact_rows(const DModel& m, const WorkRows& R, const Ro
     }
 }
 
-// Staging of one contact row (see RowJac): the columns of its two links' chains, entry p of the lane's row in its tile
-// column.
-struct GroupJac {
-    float* col;                // the lane's tile column
-    const uint32_t* chains;    // [4 * link + k]: dofs of the link and of its ancestors
+// a staged row written as its group's columns
+struct GroupJac : ChainJac {
     const DModel& m;
     const RowGroups& Q;
-    uint32_t& m0;
-    uint32_t& m1;
-    uint32_t& m2;
-    uint32_t& m3;
-    template <class R>
-    __device__ __forceinline__ void begin(const R&, int, int, int la, int lb) const {
-        m0 = chains[4 * la];
-        m1 = chains[4 * la + 1];
-        m2 = chains[4 * la + 2];
-        m3 = chains[4 * la + 3];
-        if (lb > -1) {
-            m0 |= chains[4 * lb];
-            m1 |= chains[4 * lb + 1];
-            m2 |= chains[4 * lb + 2];
-            m3 |= chains[4 * lb + 3];
-        }
-        for (int p = 0; p < Q.W; p++) col[p * kTileStride] = 0.f;
-    }
-    template <class R>
-    __device__ __forceinline__ float& at(const R&, int, int k) const {
-        const uint32_t below = (1u << (k & 31)) - 1;
-        const int w = k >> 5;
-        int p = __popc((w == 0 ? m0 : w == 1 ? m1 : w == 2 ? m2 : m3) & below);
-        if (w > 0) p += __popc(m0);
-        if (w > 1) p += __popc(m1);
-        if (w > 2) p += __popc(m2);
-        return col[p * kTileStride];
-    }
+    __device__ __forceinline__ GroupJac(float* col, const uint32_t* chains, const DModel& model, const RowGroups& groups)
+        : ChainJac{col, chains, groups.W, 0, 0, 0, 0}, m(model), Q(groups) {}
     template <class R>
     __device__ __forceinline__ void flush(const R&, int c, int D) const {
         for (int p = 0; p < Q.W; p += 4)
@@ -159,17 +129,17 @@ struct GroupJac {
                                                                 col[(p + 2) * kTileStride], col[(p + 3) * kTileStride]);
         const int g = Q.group(c);
         if (((c - Q.n1) & 3) != 0) return;  // the first of the contact's four rows writes what they share
-        uint64_t lo = m0 | (uint64_t)m1 << 32, hi = m2 | (uint64_t)m3 << 32;
+        uint64_t l = lo(), h = hi();
         *(uint4*)(Q.mask + 4 * (size_t)g) = make_uint4(m0, m1, m2, m3);
-        Q.ent[g] = group_entities(m, lo, hi);
+        Q.ent[g] = group_entities(m, l, h);
         for (int p = 0; p < Q.W; p++) {
             int d = D;
-            if (lo) {
-                d = __builtin_ctzll(lo);
-                lo &= lo - 1;
-            } else if (hi) {
-                d = kWave + __builtin_ctzll(hi);
-                hi &= hi - 1;
+            if (l) {
+                d = __builtin_ctzll(l);
+                l &= l - 1;
+            } else if (h) {
+                d = kWave + __builtin_ctzll(h);
+                h &= h - 1;
             }
             Q.idx[(size_t)g * Q.W + p] = (uint8_t)d;
         }
@@ -178,9 +148,9 @@ struct GroupJac {
 
 // solver.py:580-1286: equality, friction-loss and limit rows uniformly (few rows), contact rows one lane per row.
 // tile: max(W, kTileMinRows) tile rows, then 4 words per link.
-__device__ inline void island_constraints(const DModel& m, const LState& loc, const DState& st, int b,
+__device__ __forceinline__ void island_constraints(const DModel& m, const LState& loc, const DState& st, int b,
                                           const WorkRows& R, RowGroups& Q, int lane, float* tile) {
-    const int D = m.D, L = m.L;
+    const int D = m.D;
     const DenseRows dr{Q.dense, R, 0, D};
     int nc = equality_rows(m, loc, 0, dr);
     const int neq = nc;
@@ -192,25 +162,8 @@ __device__ inline void island_constraints(const DModel& m, const LState& loc, co
     Q.ncont = m.enable_collision ? LF(n_contacts, 0) : 0;
     if (Q.ncont > 0) {
         uint32_t* chains = (uint32_t*)(tile + island_tile_rows(Q.W) * kTileStride);
-        for (int l = lane; l < L; l += kWave) {
-            uint32_t w0 = 0, w1 = 0, w2 = 0, w3 = 0;
-            for (int k = l; k > -1; k = m.link_parent[k])
-                for (int d = m.link_dof_start[k]; d < m.link_dof_end[k]; d++) {
-                    const uint32_t bit = 1u << (d & 31);
-                    const int w = d >> 5;
-                    w0 |= w == 0 ? bit : 0;
-                    w1 |= w == 1 ? bit : 0;
-                    w2 |= w == 2 ? bit : 0;
-                    w3 |= w == 3 ? bit : 0;
-                }
-            chains[4 * l] = w0;
-            chains[4 * l + 1] = w1;
-            chains[4 * l + 2] = w2;
-            chains[4 * l + 3] = w3;
-        }
-        wave_sync();
-        uint32_t m0, m1, m2, m3;
-        const GroupJac gj{tile + lane, chains, m, Q, m0, m1, m2, m3};
+        link_chains(m, chains, lane);
+        const GroupJac gj(tile + lane, chains, m, Q);
         for (int r = lane; r < 4 * Q.ncont; r += kWave)
             contact_row(m, loc, 0, st, b, R, r >> 2, r & 3, nc, gj);
         nc += 4 * Q.ncont;
@@ -248,7 +201,7 @@ struct IslandDofs {
 
 // Islands: every group joins its entities; labels (the smallest first dof of an entity reached) spread over the groups
 // until none changes. lds: island_words(D) words.
-__device__ inline void find_islands(const DModel& m, const RowGroups& Q, int n_groups, int lane, int* lds,
+__device__ __forceinline__ void find_islands(const DModel& m, const RowGroups& Q, int n_groups, int lane, int* lds,
                                     IslandDofs& I) {
     const int D = m.D;
     int* lab = lds;
@@ -392,8 +345,11 @@ __device__ inline void find_islands(const DModel& m, const RowGroups& Q, int n_g
     wave_sync();
 }
 
-// The solver's state on a lane: its dofs' vectors, and the sums of the line search.
-template <bool kHLds>
+// The solver's state on a lane: its dofs' vectors, and the sums of the line search. Rows of up to 4 kQ entries. One
+// wavefront per SIMD is all a batch of 1024 gives, so nothing hides a load but other loads: the loops below load what
+// they need for both of a lane's dofs, for several rows, or one step ahead, before they use any of it (Hessian 120 k ->
+// 81 k cycles a call, factor 36 k -> 35 k, line search 29 k -> 21 k, row builder 250 k -> 113 k on 1024 box piles).
+template <bool kHLds, int kQ>
 struct IslandSolver {
     const DModel& m;
     const LState& loc;
@@ -403,6 +359,8 @@ struct IslandSolver {
     float* H;  // the islands' packed triangles, first the Hessian, then its factor
     float* xv; // vector in position order: D + 1 words, xv[D] = 0
     int lane, nc, ne, nef;
+    static constexpr int kRows = kQ <= 3 ? 5 : 1;     // rows of a lane taken together
+    static constexpr int kQuads = kQ <= 3 ? kQ : 1;   // quads of a row taken together
     float qacc[2], Ma[2], force[2], acc0[2], qfc[2], grad[2], Mgrad[2], search[2], mv[2];
     float gauss, qg[3], es[3];
 
@@ -426,29 +384,53 @@ struct IslandSolver {
             out[h] = seq_sum<6>(0.f, I.e0[h], I.e1[h], [&](int j) { return row[j] * x[j]; });
         }
     }
-    // J x + init for row c, in column order, x in xv
-    __device__ __forceinline__ float row_dot(int c, float init) const {
+    // out[u] = init[u] + J x for rows c0 + lane + 64 u (the last row again past the end), in column order, x in xv
+    template <int U>
+    __device__ __forceinline__ void row_dots(int c0, float (&out)[U]) const {
         const int W = Q.W;
-        const float4* j = (const float4*)(Q.J + (size_t)c * W);
-        const uint32_t* ix = (const uint32_t*)(Q.idx + (size_t)Q.group(c) * W);
-        float4 v[kRowWidthMax / 4];
-        uint32_t k[kRowWidthMax / 4];
+        for (int q0 = 0; 4 * q0 < W; q0 += kQuads) {
+            float4 v[U][kQuads];
+            uint32_t k[U][kQuads];
 #pragma unroll
-        for (int q = 0; q < kRowWidthMax / 4; q++)
-            if (4 * q < W) {
-                v[q] = j[q];
-                k[q] = ix[q];
-            }
-        float s = init;
+            for (int u = 0; u < U; u++) {
+                const int c = min(c0 + u * kWave + lane, nc - 1);
+                const float4* j = (const float4*)(Q.J + (size_t)c * W) + q0;
+                const uint32_t* ix = (const uint32_t*)(Q.idx + (size_t)Q.group(c) * W) + q0;
 #pragma unroll
-        for (int q = 0; q < kRowWidthMax / 4; q++)
-            if (4 * q < W) {
-                s = s + v[q].x * xv[k[q] & 0xff];
-                s = s + v[q].y * xv[(k[q] >> 8) & 0xff];
-                s = s + v[q].z * xv[(k[q] >> 16) & 0xff];
-                s = s + v[q].w * xv[k[q] >> 24];
+                for (int q = 0; q < kQuads; q++) {  // past the row's last quad: that quad again, left out below
+                    const int qq = min(q, W / 4 - 1 - q0);
+                    v[u][q] = j[qq];
+                    k[u][q] = ix[qq];
+                }
             }
-        return s;
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int q = 0; q < kQuads; q++)
+                    if (4 * (q0 + q) < W) {
+                        out[u] = out[u] + v[u][q].x * xv[k[u][q] & 0xff];
+                        out[u] = out[u] + v[u][q].y * xv[(k[u][q] >> 8) & 0xff];
+                        out[u] = out[u] + v[u][q].z * xv[(k[u][q] >> 16) & 0xff];
+                        out[u] = out[u] + v[u][q].w * xv[k[u][q] >> 24];
+                    }
+        }
+    }
+    // Jaref = J qacc - aref, qacc in xv
+    __device__ __forceinline__ void init_rows() const {
+        for (int c0 = 0; c0 < nc; c0 += kRows * kWave) {
+            float s[kRows];
+#pragma unroll
+            for (int u = 0; u < kRows; u++) s[u] = -R.aref(min(c0 + u * kWave + lane, nc - 1));
+            row_dots(c0, s);
+#pragma unroll
+            for (int u = 0; u < kRows; u++)
+                if (c0 + u * kWave + lane < nc) R.Jaref(c0 + u * kWave + lane) = s[u];
+        }
+        wave_sync();
+    }
+    // the k-th group of this lane's dof h; any valid entry (the environment's first group) when there is none
+    __device__ __forceinline__ int entry(int h, int k) const {
+        return k < I.cnt[h] ? Q.list[(size_t)k * m.D + lane + h * kWave] : 0;
     }
     __device__ __forceinline__ float dof_sum(float a, float b) const {
         return wave_sum_f((I.own[0] ? a : 0.f) + (I.own[1] ? b : 0.f));
@@ -492,29 +474,30 @@ struct IslandSolver {
             }
         }
         wave_sync();
+        qfc[0] = qfc[1] = 0.f;
+        const int most = max(I.cnt[0], I.cnt[1]);
+        int e[2] = {entry(0, 0), entry(1, 0)};
+        for (int k = 0; k < most; k++) {
+            float v[2][4], f[2][4];
+            const int en[2] = {entry(0, k + 1), entry(1, k + 1)};
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            float s = 0.f;
-            if (I.own[h]) {
-                const int* li = Q.list + lane + h * kWave;
-                for (int k = 0; k < I.cnt[h]; k++) {
-                    const int e = li[(size_t)k * m.D], g = e >> 5, p = e & 31, c = Q.row0(g);
-                    const float* j = Q.J + (size_t)c * Q.W + p;
-                    if (Q.four(g)) {
-                        float v[4], f[4];
+            for (int h = 0; h < 2; h++) {
+                const int g = e[h] >> 5, c = Q.row0(g), last = Q.four(g) ? 3 : 0;
+                const float* j = Q.J + (size_t)c * Q.W + (e[h] & 31);
 #pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            v[r] = j[r * Q.W];
-                            f[r] = R.force(c + r);
-                        }
-#pragma unroll
-                        for (int r = 0; r < 4; r++) s = s + v[r] * f[r];
-                    } else {
-                        s = s + j[0] * R.force(c);
-                    }
+                for (int r = 0; r < 4; r++) {
+                    v[h][r] = j[min(r, last) * Q.W];
+                    f[h][r] = R.force(c + min(r, last));
                 }
             }
-            qfc[h] = s;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const bool four = Q.four(e[h] >> 5);
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (k < I.cnt[h] && (r == 0 || four)) qfc[h] = qfc[h] + v[h][r] * f[h][r];
+                e[h] = en[h];
+            }
         }
         float cost = wave_sum_f(pf);
         gauss = dof_sum(0.5f * (Ma[0] - force[0]) * (qacc[0] - acc0[0]), 0.5f * (Ma[1] - force[1]) * (qacc[1] - acc0[1]));
@@ -524,50 +507,98 @@ struct IslandSolver {
     // solver.py:1395-1452: the lower triangle's row of each of this lane's dofs, its groups in order
     __device__ __forceinline__ void hessian() const {
         const float eps = m.eps;
+        const int W = Q.W;
         wave_sync();
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            if (!I.own[h]) continue;
-            const int d = lane + h * kWave, W = Q.W;
-            float* row = H + I.hb[h];
-            for (int j = 0; j <= I.li[h]; j += 4) *(float4*)(row + j) = make_float4(0.f, 0.f, 0.f, 0.f);
-            float* at = row + I.li[h] - I.pos[h];  // the island's position 0 in this row
-            const int* li = Q.list + d;
-            for (int k = 0; k < I.cnt[h]; k++) {
-                const int e = li[(size_t)k * m.D], g = e >> 5, p = e & 31, c = Q.row0(g), nr = Q.four(g) ? 4 : 1;
+        for (int h = 0; h < 2; h++)
+            if (I.own[h])
+                for (int j = 0; j <= I.li[h]; j += 4) *(float4*)(H + I.hb[h] + j) = make_float4(0.f, 0.f, 0.f, 0.f);
+        const int most = max(I.cnt[0], I.cnt[1]);
+        int e[2] = {entry(0, 0), entry(1, 0)};
+        for (int k = 0; k < most; k++) {
+            float ji[2][4], Dc[2][4];
+            int act[2][4];
+            const int en[2] = {entry(0, k + 1), entry(1, k + 1)};
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int g = e[h] >> 5, p = e[h] & 31, c = Q.row0(g), last = Q.four(g) ? 3 : 0;
                 const float* J = Q.J + (size_t)c * W;
-                float ji[4], Dc[4], act[4];
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    ji[r] = 0.f;
-                    Dc[r] = act[r] = 0.f;
-                    if (r < nr) {
-                        ji[r] = J[r * W + p];
-                        Dc[r] = R.efc_D(c + r);
-                        act[r] = (float)R.active(c + r);
+                    const int rr = min(r, last);
+                    ji[h][r] = J[rr * W + p];
+                    Dc[h][r] = R.efc_D(c + rr);
+                    act[h][r] = R.active(c + rr);
+                }
+            }
+            // kQuads columns' quads at a time
+            for (int q0 = 0; 4 * q0 < W; q0 += kQuads) {
+                uint32_t ix[2][kQuads];
+                float4 v[2][kQuads][4];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int g = e[h] >> 5, c = Q.row0(g), last = Q.four(g) ? 3 : 0;
+                    const float* J = Q.J + (size_t)c * W + 4 * q0;
+                    const uint8_t* id = Q.idx + (size_t)g * W + 4 * q0;
+#pragma unroll
+                    for (int q = 0; q < kQuads; q++) {  // past the row's last quad: that quad again, never used
+                        const int qq = 4 * min(q, W / 4 - 1 - q0);
+                        ix[h][q] = *(const uint32_t*)(id + qq);
+#pragma unroll
+                        for (int r = 0; r < 4; r++) v[h][q][r] = *(const float4*)(J + min(r, last) * W + qq);
                     }
                 }
-                for (int q = 0; q <= p; q += 4) {
-                    const uint32_t ix = *(const uint32_t*)(Q.idx + (size_t)g * W + q);
-                    float4 v[4];
 #pragma unroll
-                    for (int r = 0; r < 4; r++) v[r] = *(const float4*)(J + (r < nr ? r : 0) * W + q);
+                for (int h = 0; h < 2; h++) {
+                    const int p = e[h] & 31;
+                    if (k >= I.cnt[h] || 4 * q0 > p) continue;
+                    const bool four = Q.four(e[h] >> 5);
+                    float* row = H + I.hb[h];
+                    float* at = row + I.li[h] - I.pos[h];  // the island's position 0 in this row
 #pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        if (q + u > p) continue;
-                        float* s = at + ((ix >> (8 * u)) & 0xff);
-                        float x = *s;
+                    for (int q = 0; q < kQuads; q++) {
+                        const int n = p - 4 * (q0 + q);  // columns 0 .. n of the quad are at or left of the dof
+                        if (n < 0) continue;
+                        float* s[4];
+                        float x[4];
 #pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            const float jj = u == 0 ? v[r].x : u == 1 ? v[r].y : u == 2 ? v[r].z : v[r].w;
-                            if (fabsf(ji[r]) > eps) x = x + jj * ji[r] * Dc[r] * act[r];
+                        for (int u = 0; u < 4; u++) {
+                            s[u] = u <= n ? at + ((ix[h][q] >> (8 * u)) & 0xff) : row;
+                            x[u] = *s[u];
                         }
-                        *s = x;
+#pragma unroll
+                        for (int u = 0; u < 4; u++) {
+#pragma unroll
+                            for (int r = 0; r < 4; r++) {
+                                const float4 w = v[h][q][r];
+                                const float jj = u == 0 ? w.x : u == 1 ? w.y : u == 2 ? w.z : w.w;
+                                const float t = jj * ji[h][r] * Dc[h][r] * (float)act[h][r];
+                                if (fabsf(ji[h][r]) > eps && (r == 0 || four)) x[u] = x[u] + t;
+                            }
+                        }
+#pragma unroll
+                        for (int u = 0; u < 4; u++)
+                            if (u <= n) *s[u] = x[u];
                     }
                 }
             }
+            e[0] = en[0];
+            e[1] = en[1];
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if (!I.own[h]) continue;
+            const int d = lane + h * kWave;
             const float* mass = FP(loc, mass_mat) + (size_t)d * m.D;
-            for (int j = I.e0[h]; j <= d; j++) row[I.li[h] - d + j] = row[I.li[h] - d + j] + mass[j];
+            float* row = H + I.hb[h] + I.li[h] - d;
+            int j = I.e0[h];
+            for (; j + 3 <= d + 1; j += 3) {
+                const float a = mass[j], b = mass[j + 1], c = mass[j + 2];
+                row[j] = row[j] + a;
+                row[j + 1] = row[j + 1] + b;
+                row[j + 2] = row[j + 2] + c;
+            }
+            for (; j <= d; j++) row[j] = row[j] + mass[j];
         }
         wave_sync();
     }
@@ -576,40 +607,71 @@ struct IslandSolver {
     // pivot t of its island forms the pivot and its own entry (the sums over k in order)
     __device__ __forceinline__ void factor() const {
         for (int t = 0; t < I.steps; t++) {
-            float val[2];
+            const bool on[2] = {I.own[0] && I.li[0] >= t, I.own[1] && I.li[1] >= t};
+            float val[2] = {0.f, 0.f};
+            if (on[0] || on[1]) {
+                const float *Lk[2], *Lr[2];
+                float s[2], hr[2], dt[2] = {0.f, 0.f};
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                val[h] = 0.f;
-                if (!(I.own[h] && I.li[h] >= t)) continue;
-                const float* Lk = H + I.cb[h] + tri4(t);
-                const float* Lr = H + I.hb[h];
-                float s = Lk[t], dt = 0.f;
-                const float hr = Lr[t];
+                for (int h = 0; h < 2; h++) {  // a dof with nothing to do repeats the lane's other one
+                    const int g = on[h] ? h : 1 - h;
+                    Lk[h] = H + (g ? I.cb[1] : I.cb[0]) + tri4(t);
+                    Lr[h] = H + (g ? I.hb[1] : I.hb[0]);
+                    s[h] = Lk[h][t];
+                    hr[h] = Lr[h][t];
+                }
                 int j = 0;
                 for (; j + 4 <= t; j += 4) {
-                    const float4 a = *(const float4*)(Lk + j), c = *(const float4*)(Lr + j);
-                    s = s - a.x * a.x;
-                    s = s - a.y * a.y;
-                    s = s - a.z * a.z;
-                    s = s - a.w * a.w;
-                    dt = dt + c.x * a.x;
-                    dt = dt + c.y * a.y;
-                    dt = dt + c.z * a.z;
-                    dt = dt + c.w * a.w;
+                    float4 a[2], c[2];
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        a[h] = *(const float4*)(Lk[h] + j);
+                        c[h] = *(const float4*)(Lr[h] + j);
+                    }
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        s[h] = s[h] - a[h].x * a[h].x;
+                        s[h] = s[h] - a[h].y * a[h].y;
+                        s[h] = s[h] - a[h].z * a[h].z;
+                        s[h] = s[h] - a[h].w * a[h].w;
+                        dt[h] = dt[h] + c[h].x * a[h].x;
+                        dt[h] = dt[h] + c[h].y * a[h].y;
+                        dt[h] = dt[h] + c[h].z * a[h].z;
+                        dt[h] = dt[h] + c[h].w * a[h].w;
+                    }
                 }
-                for (; j < t; j++) {
-                    const float a = Lk[j];
-                    s = s - a * a;
-                    dt = dt + Lr[j] * a;
+                if (j < t) {  // the row's last, partly filled quad
+                    float4 a[2], c[2];
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        a[h] = *(const float4*)(Lk[h] + j);
+                        c[h] = *(const float4*)(Lr[h] + j);
+                    }
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        s[h] = s[h] - a[h].x * a[h].x;
+                        dt[h] = dt[h] + c[h].x * a[h].x;
+                        if (j + 1 < t) {
+                            s[h] = s[h] - a[h].y * a[h].y;
+                            dt[h] = dt[h] + c[h].y * a[h].y;
+                        }
+                        if (j + 2 < t) {
+                            s[h] = s[h] - a[h].z * a[h].z;
+                            dt[h] = dt[h] + c[h].z * a[h].z;
+                        }
+                    }
                 }
-                const float dii = sqrtf(fmaxf(s, m.eps));
-                const float inv = 1.f / dii;
-                val[h] = I.li[h] == t ? dii : (hr - dt) * inv;
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const float dii = sqrtf(fmaxf(s[h], m.eps));
+                    const float inv = 1.f / dii;
+                    val[h] = I.li[h] == t ? dii : (hr[h] - dt[h]) * inv;
+                }
             }
             wave_sync();
 #pragma unroll
             for (int h = 0; h < 2; h++)
-                if (I.own[h] && I.li[h] >= t) H[I.hb[h] + t] = val[h];
+                if (on[h]) H[I.hb[h] + t] = val[h];
             wave_sync();
         }
     }
@@ -617,42 +679,57 @@ struct IslandSolver {
     // solver.py:2722-2751 + :1893-1910: Mgrad = (L L^T)^-1 grad, column by column, all islands side by side
     __device__ __forceinline__ void newton_direction() {
         float cur[2], dg[2];
+        int x0[2];  // the island's first position
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             cur[h] = grad[h];
             dg[h] = I.own[h] ? H[I.hb[h] + I.li[h]] : 1.f;
+            x0[h] = I.pos[h] - I.li[h];
         }
+        auto below = [&](int h, int t) { return (I.own[h] && I.li[h] > t) ? H[I.hb[h] + t] : 0.f; };
+        auto beside = [&](int h, int t) {
+            return (I.own[h] && I.li[h] < t && t < I.n[h]) ? H[I.cb[h] + tri4(t) + I.li[h]] : 0.f;
+        };
         wave_sync();
+        float l[2] = {below(0, 0), below(1, 0)};
         for (int t = 0; t < I.steps; t++) {
-            float l[2];
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                l[h] = (I.own[h] && I.li[h] > t) ? H[I.hb[h] + t] : 0.f;
-                if (I.own[h] && I.li[h] == t) {
-                    cur[h] = cur[h] / dg[h];
-                    xv[I.pos[h]] = cur[h];
-                }
-            }
-            wave_sync();
+            const float ln[2] = {below(0, t + 1), below(1, t + 1)};
+            const float c[2] = {cur[0] / dg[0], cur[1] / dg[1]};
 #pragma unroll
             for (int h = 0; h < 2; h++)
-                if (I.own[h] && I.li[h] > t) cur[h] = cur[h] - l[h] * xv[I.pos[h] - I.li[h] + t];
+                if (I.own[h] && I.li[h] == t) xv[I.pos[h]] = cur[h] = c[h];
+            wave_sync();
+            float x[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) x[h] = (I.own[h] && I.li[h] > t) ? xv[x0[h] + t] : 0.f;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                if (I.own[h] && I.li[h] > t) cur[h] = cur[h] - l[h] * x[h];
+                l[h] = ln[h];
+            }
             wave_sync();
         }
+        l[0] = beside(0, I.steps - 1);
+        l[1] = beside(1, I.steps - 1);
         for (int t = I.steps - 1; t >= 0; t--) {
-            float l[2];
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                l[h] = (I.own[h] && I.li[h] < t && t < I.n[h]) ? H[I.cb[h] + tri4(t) + I.li[h]] : 0.f;
-                if (I.own[h] && I.li[h] == t) {
-                    cur[h] = cur[h] / dg[h];
-                    xv[I.pos[h]] = cur[h];
-                }
-            }
-            wave_sync();
+            const float ln[2] = {beside(0, t - 1), beside(1, t - 1)};
+            const float c[2] = {cur[0] / dg[0], cur[1] / dg[1]};
 #pragma unroll
             for (int h = 0; h < 2; h++)
-                if (I.own[h] && I.li[h] < t && t < I.n[h]) cur[h] = cur[h] - l[h] * xv[I.pos[h] - I.li[h] + t];
+                if (I.own[h] && I.li[h] == t) xv[I.pos[h]] = cur[h] = c[h];
+            wave_sync();
+            float x[2];
+            bool on[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                on[h] = I.own[h] && I.li[h] < t && t < I.n[h];
+                x[h] = on[h] ? xv[x0[h] + t] : 0.f;
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                if (on[h]) cur[h] = cur[h] - l[h] * x[h];
+                l[h] = ln[h];
+            }
             wave_sync();
         }
 #pragma unroll
@@ -692,28 +769,41 @@ struct IslandSolver {
         qg[1] = dof_sum(search[0] * Ma[0] - search[0] * force[0], search[1] * Ma[1] - search[1] * force[1]);
         qg[2] = dof_sum(0.5f * search[0] * mv[0], 0.5f * search[1] * mv[1]);
         float t[3] = {0.f, 0.f, 0.f}, e[3] = {0.f, 0.f, 0.f};
-        for (int c = lane; c < nc; c += kWave) {
-            const float ja = R.Jaref(c), Dc = R.efc_D(c);
-            const float jv = row_dot(c, 0.f);
-            R.jv(c) = jv;
-            float f0 = Dc * (0.5f * ja * ja), f1 = Dc * (jv * ja), f2 = Dc * (0.5f * jv * jv);
-            if (c < ne) {
-                e[0] = e[0] + f0;
-                e[1] = e[1] + f1;
-                e[2] = e[2] + f2;
-            } else if (c < nef) {
-                const float f = R.fl(c), rf = R.diag(c) * f;
-                const bool ln = ja <= -rf, lp = ja >= rf;
-                if (ln || lp) friction_line(f, rf, ja, jv, ln, lp, f0, f1, f2);
-            } else {
-                const float a = (float)(ja < 0.f);
-                f0 = f0 * a;
-                f1 = f1 * a;
-                f2 = f2 * a;
+        for (int c0 = 0; c0 < nc; c0 += kRows * kWave) {
+            float jr[kRows], dr[kRows], vr[kRows];
+#pragma unroll
+            for (int u = 0; u < kRows; u++) {
+                const int c = min(c0 + u * kWave + lane, nc - 1);
+                jr[u] = R.Jaref(c);
+                dr[u] = R.efc_D(c);
+                vr[u] = 0.f;
             }
-            t[0] = t[0] + f0;
-            t[1] = t[1] + f1;
-            t[2] = t[2] + f2;
+            row_dots(c0, vr);
+#pragma unroll
+            for (int u = 0; u < kRows; u++) {
+                const int c = c0 + u * kWave + lane;
+                if (c >= nc) continue;
+                const float ja = jr[u], Dc = dr[u], jv = vr[u];
+                R.jv(c) = jv;
+                float f0 = Dc * (0.5f * ja * ja), f1 = Dc * (jv * ja), f2 = Dc * (0.5f * jv * jv);
+                if (c < ne) {
+                    e[0] = e[0] + f0;
+                    e[1] = e[1] + f1;
+                    e[2] = e[2] + f2;
+                } else if (c < nef) {
+                    const float f = R.fl(c), rf = R.diag(c) * f;
+                    const bool ln = ja <= -rf, lp = ja >= rf;
+                    if (ln || lp) friction_line(f, rf, ja, jv, ln, lp, f0, f1, f2);
+                } else {
+                    const float a = (float)(ja < 0.f);
+                    f0 = f0 * a;
+                    f1 = f1 * a;
+                    f2 = f2 * a;
+                }
+                t[0] = t[0] + f0;
+                t[1] = t[1] + f1;
+                t[2] = t[2] + f2;
+            }
         }
 #pragma unroll
         for (int k = 0; k < 3; k++) {
@@ -787,14 +877,14 @@ struct IslandSolver {
 
 // solver.py:2936-3059 (init), :3063-3139 (Newton or conjugate-gradient iteration), :3164-3190 (body), :3241-3261,
 // :3199-3237. tile: at least island_words(D) words; H: the packed triangles (LDS, or the record's nt_H).
-template <bool kHLds>
-__device__ inline void island_solve(const DModel& m, const LState& loc, const DState& st, int b, const WorkRows& R,
+template <bool kHLds, int kQ>
+__device__ __forceinline__ void island_solve_rows(const DModel& m, const LState& loc, const DState& st, int b, const WorkRows& R,
                                     const RowGroups& Q, int lane, float* tile, float* H) {
     const int D = m.D;
     const int nc = LF(n_con, 0), ne = LF(n_con_eq, 0), nef = ne + LF(n_con_fl, 0);
     IslandDofs I;
     find_islands(m, Q, nc - 3 * Q.ncont, lane, (int*)tile, I);
-    IslandSolver<kHLds> S{m, loc, R, Q, I, H, tile, lane, nc, ne, nef};
+    IslandSolver<kHLds, kQ> S{m, loc, R, Q, I, H, tile, lane, nc, ne, nef};
     const bool ws = nc > 0 && LF(is_warmstart, 0);
 #pragma unroll
     for (int h = 0; h < 2; h++) {
@@ -809,8 +899,7 @@ __device__ inline void island_solve(const DModel& m, const LState& loc, const DS
     if (lane == 0) S.xv[D] = 0.f;
     S.put(S.qacc);
     S.mass_mul(S.Ma);
-    for (int c = lane; c < nc; c += kWave) R.Jaref(c) = S.row_dot(c, -R.aref(c));
-    wave_sync();
+    S.init_rows();
     const bool cg = m.solver_type == RS_SOLVER_CG;
     float prev = LF(cost, 0);
     float cost = S.update(true, 0.f);
@@ -902,6 +991,14 @@ __device__ inline void island_solve(const DModel& m, const LState& loc, const DS
     wave_sync();
     export_row_forces(m, loc, st, b, R, lane);
     wave_sync();
+}
+
+// rows of up to 12 entries (free bodies and short chains) hold all their loads in registers; longer ones take fewer at once
+template <bool kHLds>
+__device__ __forceinline__ void island_solve(const DModel& m, const LState& loc, const DState& st, int b, const WorkRows& R,
+                                    const RowGroups& Q, int lane, float* tile, float* H) {
+    if (Q.W <= 12) island_solve_rows<kHLds, 3>(m, loc, st, b, R, Q, lane, tile, H);
+    else island_solve_rows<kHLds, kRowWidthMax / 4>(m, loc, st, b, R, Q, lane, tile, H);
 }
 
 #undef LF

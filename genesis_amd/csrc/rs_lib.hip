@@ -88,7 +88,17 @@ struct rs_graph {
 
 static int64_t work_floats(const rs_model_header& h, int row_width);
 
-// row_width: the island solver's row width (RS_N_WORK depends on it)
+// Whether a model with short rows takes the island solver. Its results differ from the dense solver's in the last bits,
+// as those of any two orders of summing do, and a contact that a detection finds or misses by a last bit moves its
+// environment visibly. MPR's perturbed box-box detections have such edges all the time (a resting pile of 20 boxes: one
+// environment in 200 within four steps), so models with them keep the dense solver's sums, bit for bit, at 2.3 times the
+// island solver's time. The separating-axis test meets one in 7000 environments of stacked boxes within four steps and
+// none in 14000 of a resting pile; models with no collision pairs have none.
+static bool takes_islands(const rs_model_header& h, int row_width) {
+    return row_width > 0 && (h.box_box_detection || !h.enable_collision || h.n_pairs == 0);
+}
+
+// row_width: the model's row width (RS_N_WORK depends on it)
 static int64_t count_of(const rs_model_header& h, int kind, int row_width = 0) {
     switch (kind) {
         case RS_N_ONE: return 1;
@@ -145,13 +155,14 @@ static void fused_layout(const rs_model_header& h, FusedArgs* fa, int row_width)
     fa->lds_wave = (int)up4((int64_t)kTileStride * tile_rows(h.n_dofs));
     fa->sched = 0;
     fa->row_width = row_width;
+    fa->islands = takes_islands(h, row_width);
     fa->h_off = -1;
     const int64_t C = h.len_constraints > 0 ? h.len_constraints : 1, D = h.n_dofs;
     fa->off_loc = 0;
     fa->off_jac = (int)up4(off);
     // the jacobian rows: dense, or the island solver's row groups (rs_island_solver.h row_groups)
     int64_t jac = up4(C * D);
-    if (row_width > 0) {
+    if (fa->islands) {
         const int64_t G = row_group_max(h.n_equalities, h.n_dofs, h.max_contact_pairs);
         jac = std::max(jac, up4(C * row_width + G * (row_width / 4 + 5 + D) + (6 * (int64_t)h.n_equalities + D) * D));
     }
@@ -165,8 +176,8 @@ static void fused_layout(const rs_model_header& h, FusedArgs* fa, int row_width)
     fa->work_stride = (total + 63) / 64 * 64;
 }
 
-// LDS slice of one wavefront: the private region (when it is in LDS) followed by the row tile (the island solver's: its
-// tile rows and four words per link)
+// LDS slice of one wavefront: the private region (when it is in LDS) followed by the row tile (models with short rows: the
+// tile rows that stage one and four words per link)
 static int tile_floats(const rs_model_header& h, const FusedArgs& fa) {
     if (fa.row_width > 0) return kTileStride * island_tile_rows(fa.row_width) + 4 * h.n_links;
     return (kTileStride * tile_rows(h.n_dofs) + 3) / 4 * 4;
@@ -184,7 +195,7 @@ static int lds_slice_floats(const rs_model_header& h, const FusedArgs& fa, bool 
 // in the record's nt_H otherwise): every step of its factor and triangular solves waits for one round trip to them
 static int slice_with_triangles(const rs_model* m, const FusedArgs& fa, bool use_lds, int* h_off) {
     const int slice = lds_slice_floats(m->h, fa, use_lds), with_h = slice + tri4(m->h.n_dofs);
-    const bool in_lds = fa.row_width > 0 && (int64_t)fa.epb * with_h * 4 <= m->max_lds;
+    const bool in_lds = fa.islands && (int64_t)fa.epb * with_h * 4 <= m->max_lds;
     *h_off = in_lds ? slice : -1;
     return in_lds ? with_h : slice;
 }
@@ -484,7 +495,7 @@ static int fused_substep(const rs_model* m, const DState& st, hipStream_t s) {
     const bool lds_on = m->use_lds != 0;
     if (fa.tiled == kTileMaxDofs) launch_fused_tile16(lds_on, m->occupancy, grid, block, lds, s, m->dm, st, fa);
     else if (fa.tiled == kTileWideDofs) launch_fused_tile24(lds_on, m->occupancy, grid, block, lds, s, m->dm, st, fa);
-    else if (fa.row_width > 0) launch_fused_island(lds_on, grid, block, lds, s, m->dm, st, fa);
+    else if (fa.islands) launch_fused_island(lds_on, grid, block, lds, s, m->dm, st, fa);
     else launch_fused_generic(lds_on, grid, block, lds, s, m->dm, st, fa);
     HIP_OK(hipGetLastError());
     return RS_OK;
@@ -553,7 +564,7 @@ static bool has_convex_mesh(const rs_model_header& h, const char* blob) {
     return false;
 }
 
-// Entries per constraint row of the island solver: a row acts on at most two links, so it touches at most twice the dofs
+// Most dofs a constraint row touches: a row acts on at most two links, so it touches at most twice the dofs
 // of the longest chain of links (two for a row between joints). 0 for models that the row-tile solvers serve, with
 // more dofs than two per lane, or whose rows are longer than kRowWidthMax (a long chain: its rows are better taken as
 // dense, on the matrix cores).
@@ -645,7 +656,7 @@ int rs_model_create(const rs_model_header* h, const void* blob, size_t blob_byte
     if (hipDeviceGetAttribute(&m->n_cu, hipDeviceAttributeMultiprocessorCount, m->device) != hipSuccess) m->n_cu = 0;
     // default launch shape: two environments per workgroup (one with the island solver, whose triangles then fit in
     // LDS), private regions in LDS when they fit
-    m->fa.epb = m->fa.row_width > 0 ? 1 : 2;
+    m->fa.epb = m->fa.islands ? 1 : 2;
     m->use_lds = check_fused_config(m, m->fa, m->fa.epb, 1) == RS_OK;
     g_err.clear();
     *out = m;

@@ -29,7 +29,8 @@ struct FusedArgs {
     int gjk_words;     // LDS floats per wavefront for the GJK/EPA polytope (0: the polytope stays in the work field)
     int gjk_off;       // offset of that polytope in the wavefront's LDS slice (-1: none)
     int tile_off;      // offset of the row tile (kTileStride x tile_rows(D) floats) in the wavefront's LDS slice
-    int row_width;     // entries per constraint row of the island solver (0: the model does not use it)
+    int row_width;     // most dofs a constraint row touches, a multiple of 4 (models with 25 to 128 dofs; 0: over 32)
+    int islands;       // 1: the island solver (rs_island_solver.h)
     int h_off;         // offset of the island solver's packed triangles in the wavefront's LDS slice (-1: in nt_H)
     int sched;         // 1: map wavefronts to environments through the cost-ordered queues
     int loc_off[kMaxStateFields];  // private-region offset of each state field (local kinds only)
@@ -202,9 +203,10 @@ __device__ __forceinline__ void tile_seq_sums(float& acc, const float (&v)[NQ], 
 }
 
 // ---------------------------------------------------------------------------------------- private region
-// the local view of the environment whose private region starts at base
-__device__ __forceinline__ LState make_local(float* base, const FusedArgs& fa) {
-    return LState{base, (const RS_CONST int*)fa.loc_off};
+// the local view of the environment whose private region starts at base; off: the field offsets in constant memory (the
+// kernel-argument segment or a launch's table)
+__device__ __forceinline__ LState make_local(float* base, const RS_CONST int* off) {
+    return LState{base, off};
 }
 
 // Copy environment b's local rows between the slab and its private region, as raw 32-bit words. With env-major

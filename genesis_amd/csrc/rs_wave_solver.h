@@ -28,12 +28,16 @@ struct WorkRows {
     __device__ __forceinline__ int& active(int c) const { return ((int*)f)[(size_t)RW_ACTIVE * cap + c]; }
     __device__ __forceinline__ int& prev(int c) const { return ((int*)f)[(size_t)RW_PREV * cap + c]; }
     __device__ __forceinline__ float& tmp(int k, int c) const { return tp[(size_t)k * cap + c]; }
+    // 16-column tiles (bit t: columns 16 t ..) in which row c may hold something but zeros, for the matrix-core products
+    __device__ __forceinline__ int& tiles(int c) const { return ((int*)tp)[(size_t)(kTmpArrays - 1) * cap + c]; }
 };
+
 
 #define LF(field, row) FP(loc, field)[(row)]
 
 // a lane's column of the row tile as the staging buffer of the contact jacobian rows it builds
 struct TileJac {
+    static constexpr bool kBatch = false;
     float* col;
     __device__ __forceinline__ void begin(const WorkRows&, int, int D, int, int) const {
         for (int k = 0; k < D; k++) col[k * kTileStride] = 0.f;
@@ -44,17 +48,96 @@ struct TileJac {
     }
 };
 
+// Staging of one contact row by its columns: the dofs of its two links' chains in ascending order, entry p in the lane's
+// tile column.
+struct ChainJac {
+    static constexpr bool kBatch = true;
+    float* col;              // the lane's tile column
+    const uint32_t* chains;  // [4 * link + k]: dofs of the link and of its ancestors, 32 per word
+    int W;                   // tile rows of a staged row
+    mutable uint32_t m0, m1, m2, m3;  // the row's dofs, 32 per word (values, so that they stay in registers)
+    template <class R>
+    __device__ __forceinline__ void begin(const R&, int, int, int la, int lb) const {
+        m0 = chains[4 * la];
+        m1 = chains[4 * la + 1];
+        m2 = chains[4 * la + 2];
+        m3 = chains[4 * la + 3];
+        if (lb > -1) {
+            m0 |= chains[4 * lb];
+            m1 |= chains[4 * lb + 1];
+            m2 |= chains[4 * lb + 2];
+            m3 |= chains[4 * lb + 3];
+        }
+        for (int p = 0; p < W; p++) col[p * kTileStride] = 0.f;
+    }
+    template <class R>
+    __device__ __forceinline__ float& at(const R&, int, int k) const {
+        const uint32_t below = (1u << (k & 31)) - 1, a0 = m0, a1 = m1, a2 = m2, a3 = m3;
+        const int w = k >> 5;
+        int p = __popc(a0 & (w > 0 ? ~0u : below));
+        p += w > 0 ? __popc(a1 & (w > 1 ? ~0u : below)) : 0;
+        p += w > 1 ? __popc(a2 & (w > 2 ? ~0u : below)) : 0;
+        p += w > 2 ? __popc(a3 & below) : 0;
+        return col[p * kTileStride];
+    }
+    __device__ __forceinline__ uint64_t lo() const { return m0 | (uint64_t)m1 << 32; }
+    __device__ __forceinline__ uint64_t hi() const { return m2 | (uint64_t)m3 << 32; }
+};
+
+// the chains of ChainJac (models of at most 128 dofs)
+__device__ __forceinline__ void link_chains(const DModel& m, uint32_t* chains, int lane) {
+    for (int l = lane; l < m.L; l += kWave) {
+        uint32_t w0 = 0, w1 = 0, w2 = 0, w3 = 0;
+        for (int k = l; k > -1; k = m.link_parent[k])
+            for (int d = m.link_dof_start[k]; d < m.link_dof_end[k]; d++) {
+                const uint32_t bit = 1u << (d & 31);
+                const int w = d >> 5;
+                w0 |= w == 0 ? bit : 0;
+                w1 |= w == 1 ? bit : 0;
+                w2 |= w == 2 ? bit : 0;
+                w3 |= w == 3 ? bit : 0;
+            }
+        chains[4 * l] = w0;
+        chains[4 * l + 1] = w1;
+        chains[4 * l + 2] = w2;
+        chains[4 * l + 3] = w3;
+    }
+    wave_sync();
+}
+
+// a staged row written to its columns of a dense row that holds zeros
+struct DenseChainJac : ChainJac {
+    __device__ __forceinline__ void flush(const WorkRows& rows, int c, int) const {
+        uint64_t l = lo(), h = hi();
+        int tiles = 0;
+        for (int t = 0; t < 4; t++) {
+            tiles |= ((l >> (16 * t)) & 0xffff) ? 1 << t : 0;
+            tiles |= ((h >> (16 * t)) & 0xffff) ? 16 << t : 0;
+        }
+        rows.tiles(c) = tiles;
+        for (int p = 0; l | h; p++) {
+            const int d = l ? __builtin_ctzll(l) : kWave + __builtin_ctzll(h);
+            rows.jac(c, d) = col[p * kTileStride];
+            if (l) l &= l - 1;
+            else h &= h - 1;
+        }
+    }
+};
+
 // solver.py:580-1286: equality, friction-loss and limit rows uniformly (few rows), contact rows one lane per row (with a
-// row tile) or per contact
-__device__ inline void wave_constraints(const DModel& m, const LState& loc, const DState& st, int b, const WorkRows& R,
-                                        int lane, float* tile) {
+// row tile, or short rows: row_width > 0) or per contact. Dense rows of models with more than 24 dofs are cleared by
+// whole wavefronts and filled in their row_width columns (five stacks of four boxes x101: 261 k -> 170 k cycles a step).
+__device__ __forceinline__ void wave_constraints(const DModel& m, const LState& loc, const DState& st, int b,
+                                                 const WorkRows& R, int lane, float* tile, bool tiled, int row_width) {
     int nc = equality_rows(m, loc, 0, R);
     const int neq = nc;
     int nfl = frictionloss_rows(m, loc, 0, R, nc);
     nc += nfl;
+    if (!tiled)
+        for (int c = lane; c < nc; c += kWave) R.tiles(c) = 0xff;
     if (m.enable_collision) {
         const int ncont = LF(n_contacts, 0);
-        if (tile) {  // one lane per row: lane 4 q + i builds row i of the q-th contact of the pass
+        if (tiled) {  // one lane per row: lane 4 q + i builds row i of the q-th contact of the pass
             const TileJac jt{tile + lane};
             // rows D .. D + 2 of the tile are free until the solve: the walk's tree arrays go there when they fit
             const int D = m.D, L = m.L;
@@ -72,12 +155,24 @@ __device__ inline void wave_constraints(const DModel& m, const LState& loc, cons
             } else {
                 for (int r = lane; r < 4 * ncont; r += kWave) contact_row(m, loc, 0, st, b, R, r >> 2, r & 3, nc, jt);
             }
+        } else if (row_width > 0) {
+            uint32_t* chains = (uint32_t*)(tile + island_tile_rows(row_width) * kTileStride);
+            for (int64_t t = lane; t < (int64_t)4 * ncont * m.D; t += kWave) R.J[(size_t)nc * m.D + t] = 0.f;
+            link_chains(m, chains, lane);
+            const DenseChainJac dj{{tile + lane, chains, row_width, 0, 0, 0, 0}};
+            for (int r = lane; r < 4 * ncont; r += kWave) contact_row(m, loc, 0, st, b, R, r >> 2, r & 3, nc, dj);
         } else {
             for (int ic = lane; ic < ncont; ic += kWave) contact_rows(m, loc, 0, st, b, R, ic, nc);
+            for (int r = lane; r < 4 * ncont; r += kWave) R.tiles(nc + r) = 0xff;
         }
         nc += ncont * 4;
     }
-    if (m.enable_joint_limit) nc = limit_rows(m, loc, 0, R, nc);
+    if (m.enable_joint_limit) {
+        const int c0 = nc;
+        nc = limit_rows(m, loc, 0, R, nc);
+        if (!tiled)
+            for (int c = c0 + lane; c < nc; c += kWave) R.tiles(c) = 0xff;
+    }
     LF(n_con, 0) = nc;
     LF(n_con_eq, 0) = neq;
     LF(n_con_fl, 0) = nfl;
@@ -114,6 +209,16 @@ __device__ __forceinline__ float wave_dsum(int D, int lane, F f) {
     return wave_sum_f(p);
 }
 
+// union of the tile masks of rows c0 .. c0 + n - 1 (uniform). A product with a tile in which every row is zero adds
+// exactly nothing to its accumulators, so it is left out, loads and all: of a pile's 8 tiles a contact touches 1 to 4.
+__device__ __forceinline__ int tiles_of_rows(const WorkRows& R, int nc, int c0, int n, int lane) {
+    const int mine = lane < n && c0 + lane < nc ? R.tiles(c0 + lane) : 0;
+    int on = 0;
+#pragma unroll
+    for (int t = 0; t < kMfmaMaxDofs / 16; t++) on |= wave_ballot((mine >> t) & 1) ? 1 << t : 0;
+    return on;
+}
+
 // out[d] = sum over rows c < nc of J[c][d] w[c] (d < D <= 128) on the matrix cores: for each 16-column tile, A holds
 // the row weights (A[i][k] = w[c0 + k] for every i) and B the rows (B[k][j] = J[c0 + k][16 T + j]), so every row of
 // the tile's result is the sum; 16 rows per trip, their operands loaded before the products.
@@ -124,6 +229,7 @@ __device__ inline void gemv_t_mfma(const WorkRows& R, int nc, int D, float* out,
 #pragma unroll
     for (int t = 0; t < kMfmaMaxDofs / 16; t++) acc[t] = mfma_v4f{0.f, 0.f, 0.f, 0.f};
     for (int c0 = 0; c0 < nc; c0 += 16) {
+        const int on = tiles_of_rows(R, nc, c0, 16, lane);  // tiles where every row is zero add nothing
         float av[4], bv[4][kMfmaMaxDofs / 16];
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -131,6 +237,7 @@ __device__ inline void gemv_t_mfma(const WorkRows& R, int nc, int D, float* out,
             av[q] = c < nc ? w(c) : 0.f;
 #pragma unroll
             for (int t = 0; t < kMfmaMaxDofs / 16; t++) {
+                if (!((on >> t) & 1)) continue;
                 const int d = t * 16 + li;
                 bv[q][t] = (c < nc && d < D) ? R.jac(c, d) : 0.f;
             }
@@ -139,7 +246,7 @@ __device__ inline void gemv_t_mfma(const WorkRows& R, int nc, int D, float* out,
         for (int q = 0; q < 4; q++)
 #pragma unroll
             for (int t = 0; t < kMfmaMaxDofs / 16; t++)
-                if (t * 16 < D) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[q], bv[q][t], acc[t], 0, 0, 0);
+                if (t * 16 < D && ((on >> t) & 1)) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[q], bv[q][t], acc[t], 0, 0, 0);
     }
     if (lk == 0) {
 #pragma unroll
@@ -158,7 +265,9 @@ __device__ inline void gemv_rows_mfma(const WorkRows& R, int nc, int D, const fl
         mfma_v4f acc[4];
 #pragma unroll
         for (int q = 0; q < 4; q++) acc[q] = mfma_v4f{0.f, 0.f, 0.f, 0.f};
+        const int on = tiles_of_rows(R, nc, c0, 64, lane);
         for (int d0 = 0; d0 < D; d0 += 4) {
+            if (!((on >> (d0 >> 4)) & 1)) continue;
             const int d = d0 + lk;
             const float b = d < D ? v[d] : 0.f;
             float a[4];
@@ -311,6 +420,7 @@ __device__ inline void wave_hessian_mfma(const DModel& m, const LState& loc, con
 #pragma unroll
     for (int t = 0; t < kTiles; t++) acc[t] = mfma_v4f{0.f, 0.f, 0.f, 0.f};
     for (int c0 = 0; c0 < nc; c0 += 8) {
+        const int on = tiles_of_rows(R, nc, c0, 8, lane);
         float v[2][kT], w[2];
 #pragma unroll
         for (int s = 0; s < 2; s++) {
@@ -320,7 +430,7 @@ __device__ inline void wave_hessian_mfma(const DModel& m, const LState& loc, con
 #pragma unroll
             for (int I = 0; I < kT; I++) {
                 const int d = I * 16 + li;
-                v[s][I] = (rv && d < D) ? R.jac(c, d) : 0.f;
+                v[s][I] = ((on >> I) & 1) && rv && d < D ? R.jac(c, d) : 0.f;
             }
         }
 #pragma unroll
@@ -335,7 +445,7 @@ __device__ inline void wave_hessian_mfma(const DModel& m, const LState& loc, con
             for (int I = 0; I < kT; I++)
 #pragma unroll
                 for (int J = 0; J <= I; J++)
-                    if (I < T) acc[I * (I + 1) / 2 + J] =
+                    if (I < T && ((on >> I) & 1) && ((on >> J) & 1)) acc[I * (I + 1) / 2 + J] =
                         __builtin_amdgcn_mfma_f32_16x16x4f32(av[I], bv[J], acc[I * (I + 1) / 2 + J], 0, 0, 0);
         }
     }
@@ -467,11 +577,15 @@ __device__ inline void wave_hessian_cholesky(const DModel& m, const LState& loc,
     cholesky_in_place(D, FP(loc, nt_H), eps, lane);
 }
 
-// solver.py:1782-1822: rank-1 updates of the factor for rows whose active flag flipped, in row order;
-// returns true (uniformly) when an update degenerates
+// solver.py:1782-1822: rank-1 updates of the factor for rows whose active flag flipped, in row order; returns true
+// (uniformly) when an update degenerates. Models of up to 128 dofs: the row's vector stays in registers (lane: entries
+// lane and lane + 64), a ballot finds the next column it touches (a row touches few; every other column would be a round
+// trip to memory only to find a zero), and that column is loaded while the one before is worked on. Five stacks of four
+// boxes x101: 5.2 M -> 2.5 M cycles a step.
 __device__ inline bool wave_cholesky_incremental(const DModel& m, const LState& loc, const WorkRows& R, int lane) {
     const int D = m.D;
     const int nc = LF(n_con, 0);
+    float* H = FP(loc, nt_H);
     for (int c0 = 0; c0 < nc; c0 += kWave) {
         const int cl = c0 + lane;
         uint64_t flips = wave_ballot(cl < nc && (R.active(cl) ^ R.prev(cl)));
@@ -480,6 +594,63 @@ __device__ inline bool wave_cholesky_incremental(const DModel& m, const LState& 
             flips &= flips - 1;
             const float sign = R.active(c) ? 1.f : -1.f;
             const float sq = sqrtf(R.efc_D(c));
+            if (D <= 2 * kWave) {
+                float v[2], col[2] = {0.f, 0.f}, dk = 0.f;
+#pragma unroll
+                for (int h = 0; h < 2; h++) v[h] = lane + h * kWave < D ? R.jac(c, lane + h * kWave) * sq : 0.f;
+                int k = -1, loaded = -1;
+                for (;;) {
+                    // the next column past k that the vector touches, and the one after it as things stand
+                    uint64_t lo = wave_ballot(fabsf(v[0]) > m.eps), hi = wave_ballot(fabsf(v[1]) > m.eps);
+                    if (k >= 0) {
+                        lo = k < kWave - 1 ? lo & (~0ull << (k + 1)) : 0;
+                        if (k >= kWave) hi = k < 2 * kWave - 1 ? hi & (~0ull << (k + 1 - kWave)) : 0;
+                    }
+                    if (!(lo | hi)) break;
+                    k = lo ? __builtin_ctzll(lo) : kWave + __builtin_ctzll(hi);
+                    if (lo) lo &= lo - 1;
+                    else hi &= hi - 1;
+                    const int next = lo ? __builtin_ctzll(lo) : hi ? kWave + __builtin_ctzll(hi) : -1;
+                    if (loaded != k) {
+                        dk = H[(size_t)k * D + k];
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+                            const int i = lane + h * kWave;
+                            col[h] = i > k && i < D ? H[(size_t)i * D + k] : 0.f;
+                        }
+                    }
+                    float ncol[2] = {0.f, 0.f}, ndk = 0.f;
+                    if (next >= 0) {
+                        ndk = H[(size_t)next * D + next];
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+                            const int i = lane + h * kWave;
+                            ncol[h] = i > next && i < D ? H[(size_t)i * D + next] : 0.f;
+                        }
+                    }
+                    const float vk = readlane_f(k < kWave ? v[0] : v[1], k & (kWave - 1));
+                    const float t = dk * dk + sign * vk * vk;
+                    if (t < m.eps) return true;
+                    const float r = sqrtf(t);
+                    const float cc = r / dk, cinv = 1.f / cc, ss = vk / dk;
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const int i = lane + h * kWave;
+                        if (i > k && i < D) {
+                            const float x = (col[h] + ss * v[h] * sign) * cinv;
+                            H[(size_t)i * D + k] = x;
+                            v[h] = v[h] * cc - ss * x;
+                        } else if (i == k) {
+                            H[(size_t)k * D + k] = r;
+                        }
+                        col[h] = ncol[h];
+                    }
+                    dk = ndk;
+                    loaded = next;
+                }
+                wave_sync();
+                continue;
+            }
             for (int d = lane; d < D; d += kWave) LF(nt_vec, d) = R.jac(c, d) * sq;
             wave_sync();
             for (int k = 0; k < D; k++) {

@@ -2,7 +2,8 @@
 identical state against the per-stage step, at the sizes and orders where the island solver's bookkeeping can go wrong:
 the smallest and the largest dof count, islands of one body, of chains and of the whole model, rows of every kind
 (connect, weld, joint equality, friction loss, contact, limit), dofs in both halves of the wavefront, and the packed
-triangles in LDS (one environment per workgroup) and in the state record (two and four)."""
+triangles in LDS (one environment per workgroup) and in the state record (two and four). The same models with MPR's
+perturbed box-box contacts take the dense solver, whose row masks and rank-1 updates have the same edges."""
 
 from __future__ import annotations
 
@@ -74,12 +75,13 @@ MODELS = {
 
 
 @pytest.mark.parametrize("epb", [1, 2, 4])
+@pytest.mark.parametrize("box_box", [True, False], ids=["island", "dense"])
 @pytest.mark.parametrize("name", list(MODELS))
-def test_island_step_matches_the_per_stage_step(tmp_path, name, epb):
+def test_island_step_matches_the_per_stage_step(tmp_path, name, box_box, epb):
     from genesis_amd import runtime as rt
 
     rt.load_library()
-    model = MODELS[name](tmp_path, {})
+    model = MODELS[name](tmp_path, {"box_box_detection": box_box})
     assert 24 < model.n_dofs <= 128
     dm = rt.DeviceModel(model)
     dm.set_fused_config(epb, False, False, 0)
