@@ -421,16 +421,19 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
             wave_constraints(m, loc, st, b, R, lane, tile, kPath == 1 || kPath == 4 || (kPath == 2 && fa.tiled != 0),
                              fa.row_width);
         }
+        const SquareH square{FP(loc, nt_H), m.D};
         if constexpr (kPath == 5) {
             if (fa.h_off >= 0) island_solve<true>(m, loc, st, b, R, Q, lane, tile, slice + fa.h_off);
             else island_solve<false>(m, loc, st, b, R, Q, lane, tile, triangles_in_record(loc));
-        } else if constexpr (kPath == 1) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile);
-        else if constexpr (kPath == 4) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile);
-        else if constexpr (kPath == 0) wave_solve<0>(m, loc, st, b, R, lane, tile);
-        else if (islands) island_solve<false>(m, loc, st, b, R, Q, lane, tile, triangles_in_record(loc));
-        else if (fa.tiled == kTileMaxDofs) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile);
-        else if (fa.tiled == kTileWideDofs) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile);
-        else wave_solve<0>(m, loc, st, b, R, lane, tile);
+        } else if constexpr (kPath == 1) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile, square);
+        else if constexpr (kPath == 4) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile, square);
+        else if constexpr (kPath == 0) {
+            if (fa.h_off >= 0) wave_solve<0>(m, loc, st, b, R, lane, tile, PackedH{slice + fa.h_off});
+            else wave_solve<0>(m, loc, st, b, R, lane, tile, square);
+        } else if (islands) island_solve<false>(m, loc, st, b, R, Q, lane, tile, triangles_in_record(loc));
+        else if (fa.tiled == kTileMaxDofs) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile, square);
+        else if (fa.tiled == kTileWideDofs) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile, square);
+        else wave_solve<0>(m, loc, st, b, R, lane, tile, square);
     }
     // kernel_step_2: cacc, semi-implicit Euler, forward kinematics and velocities
     wave_update_acc<kMany>(m, loc, lane, true);

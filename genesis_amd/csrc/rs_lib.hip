@@ -191,11 +191,12 @@ static void set_lds_slice(const rs_model_header& h, FusedArgs* fa, bool use_lds,
 static int lds_slice_floats(const rs_model_header& h, const FusedArgs& fa, bool use_lds) {
     return (use_lds ? fa.loc_floats : 0) + tile_floats(h, fa) + fa.gjk_words;
 }
-// the island solver's packed triangles follow in the slice when the workgroup's slices still fit with them (they are
-// in the record's nt_H otherwise): every step of its factor and triangular solves waits for one round trip to them
+// the packed lower triangle of the Hessian of models above 24 dofs follows in the slice when the workgroup's slices still
+// fit with it (it is in nt_H otherwise): every step of a factorisation or a triangular solve waits for a round trip to it
 static int slice_with_triangles(const rs_model* m, const FusedArgs& fa, bool use_lds, int* h_off) {
     const int slice = lds_slice_floats(m->h, fa, use_lds), with_h = slice + tri4(m->h.n_dofs);
-    const bool in_lds = fa.islands && (int64_t)fa.epb * with_h * 4 <= m->max_lds;
+    const bool wanted = fa.islands || (!fa.tiled && !use_lds && m->h.n_dofs <= kMfmaMaxDofs);
+    const bool in_lds = wanted && (int64_t)fa.epb * with_h * 4 <= m->max_lds;
     *h_off = in_lds ? slice : -1;
     return in_lds ? with_h : slice;
 }
@@ -654,9 +655,9 @@ int rs_model_create(const rs_model_header* h, const void* blob, size_t blob_byte
     if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, m->device) != hipSuccess) max_lds = 0;
     m->max_lds = max_lds < 65536 ? max_lds : 65536;
     if (hipDeviceGetAttribute(&m->n_cu, hipDeviceAttributeMultiprocessorCount, m->device) != hipSuccess) m->n_cu = 0;
-    // default launch shape: two environments per workgroup (one with the island solver, whose triangles then fit in
-    // LDS), private regions in LDS when they fit
-    m->fa.epb = m->fa.islands ? 1 : 2;
+    // default launch shape: two environments per workgroup (one for models above 24 dofs, whose Hessian then fits
+    // in LDS), private regions in LDS when they fit
+    m->fa.epb = m->fa.tiled ? 2 : 1;
     m->use_lds = check_fused_config(m, m->fa, m->fa.epb, 1) == RS_OK;
     g_err.clear();
     *out = m;

@@ -31,7 +31,7 @@ struct FusedArgs {
     int tile_off;      // offset of the row tile (kTileStride x tile_rows(D) floats) in the wavefront's LDS slice
     int row_width;     // most dofs a constraint row touches, a multiple of 4 (models with 25 to 128 dofs; 0: over 32)
     int islands;       // 1: the island solver (rs_island_solver.h)
-    int h_off;         // offset of the island solver's packed triangles in the wavefront's LDS slice (-1: in nt_H)
+    int h_off;         // offset of the packed Hessian of models above 24 dofs in the wavefront's LDS slice (-1: in nt_H)
     int sched;         // 1: map wavefronts to environments through the cost-ordered queues
     int loc_off[kMaxStateFields];  // private-region offset of each state field (local kinds only)
 };

@@ -398,6 +398,20 @@ __device__ inline void cholesky_in_place(int D, float* H, float eps, int lane) {
     }
 }
 
+// Where the Hessian and its factor of a dense model (25 to 128 dofs) are: entry (i, j <= i) of a square matrix in the
+// private region, or of a packed lower triangle in LDS (rows padded to 4 words). The factorisation, its rank-1 updates
+// and the triangular solves are chains of dependent accesses, and out of LDS each link of a chain is several times
+// shorter. Five stacks of four boxes x101: 5.65 M -> 4.95 M cycles a step (Hessian and factor 812 k -> 423 k).
+struct SquareH {
+    float* p;
+    int D;
+    __device__ __forceinline__ float& at(int i, int j) const { return p[(size_t)i * D + j]; }
+};
+struct PackedH {
+    float* p;
+    __device__ __forceinline__ float& at(int i, int j) const { return p[tri4(i) + j]; }
+};
+
 // solver.py:1395-1452 (func_hessian_direct_tiled's product J^T diag(efc_D active) J) on the matrix cores, for models
 // above the row-tile classes (dense rows over many dofs): the lower triangle in 16 x 16 tiles, all accumulated
 // together over the rows 4 at a time with v_mfma_f32_16x16x4f32 (A: lane l holds J[c0 + l/16][I*16 + l%16]; B: lane l holds
@@ -405,7 +419,9 @@ __device__ inline void cholesky_in_place(int D, float* H, float eps, int lane) {
 // reference, a row's term of entry (i, j) is left out when |J[c][i]| <= EPS; the mass matrix is added afterwards on
 // blocks of one entity. The matrix cores sum the rows in their own order, so the entries differ from the
 // one-lane-per-entry sum (and from the per-stage kernels) in the last bits.
-__device__ inline void wave_hessian_mfma(const DModel& m, const LState& loc, const WorkRows& R, int lane) {
+template <class HM>
+__device__ __forceinline__ void wave_hessian_mfma(const DModel& m, const LState& loc, const WorkRows& R, const HM& H,
+                                                  int lane) {
     constexpr int kT = kMfmaMaxDofs / 16;
     constexpr int kTiles = kT * (kT + 1) / 2;  // the lower triangle's 16 x 16 tiles, (I, J <= I) in row order
     const int D = m.D;
@@ -461,7 +477,7 @@ __device__ inline void wave_hessian_mfma(const DModel& m, const LState& loc, con
                 if (i < D && j <= i) {
                     float h = acc[I * (I + 1) / 2 + J][r];
                     if (m.dof_entity[i] == m.dof_entity[j]) h = h + LF(mass_mat, i * D + j);
-                    LF(nt_H, i * D + j) = h;
+                    H.at(i, j) = h;
                 }
             }
         }
@@ -473,52 +489,82 @@ __device__ inline void wave_hessian_mfma(const DModel& m, const LState& loc, con
 // columns are factored as in cholesky_in_place for every row at or below the panel, with the sums over k starting at
 // the panel's first column (the earlier panels' terms were subtracted already), then the panel's product
 // L[rows][panel] L[cols][panel]^T is subtracted from the trailing lower triangle in 16 x 16 tiles on the matrix cores.
-// The same factor as cholesky_in_place up to the order of the sums. H: D x D row-major, lower triangle, D <= 128.
-__device__ inline void cholesky_blocked_mfma(int D, float* H, float eps, int lane) {
+// The same factor as cholesky_in_place up to the order of the sums. H: lower triangle, D <= 128. A panel is factored in
+// registers (lane: rows lane and lane + 64), its pivot row broadcast, since every column depends on the one before; a
+// tile of the product is left out where one of its factors is all zeros (it would subtract nothing: of a pile's 28 tile
+// pairs most are empty).
+template <class HM>
+__device__ __forceinline__ void cholesky_blocked_mfma(int D, const HM& H, float eps, int lane) {
     const int T = (D + 15) / 16;
     const int li = lane & 15, lk = lane >> 4;
     for (int p = 0; p < T; p++) {
         const int k0 = p * 16, k1 = min(k0 + 16, D);
-        for (int i = k0; i < k1; i++) {
-            const float* Hi = H + (size_t)i * D;
-            float hv[16];
+        const bool low = k0 < kWave;  // the pivot rows are the lanes' first rows
+        float rv[2][16], pv[16];
 #pragma unroll
-            for (int u = 0; u < 16; u++) hv[u] = k0 + u < i ? Hi[k0 + u] : 0.f;
-            float t = Hi[i];
+        for (int u = 0; u < 16; u++) {
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int r = lane + h * kWave;
+                rv[h][u] = r < D && k0 + u <= r ? H.at(r, k0 + u) : 0.f;
+            }
+            pv[u] = low ? rv[0][u] : rv[1][u];
+        }
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int i = k0 + q;
+            if (i >= k1) break;
+            float hv[16];
+            float t = readlane_f(pv[q], i & (kWave - 1));
 #pragma unroll
             for (int u = 0; u < 16; u++)
-                if (k0 + u < i) t = t - hv[u] * hv[u];
+                if (u < q) {
+                    hv[u] = readlane_f(pv[u], i & (kWave - 1));
+                    t = t - hv[u] * hv[u];
+                }
             const float dii = sqrtf(fmaxf(t, eps));
             const float inv = 1.f / dii;
-            for (int r = i + 1 + lane; r < D; r += kWave) {
-                const float* Hr = H + (size_t)r * D;
-                float rv[16];
 #pragma unroll
-                for (int u = 0; u < 16; u++) rv[u] = k0 + u < i ? Hr[k0 + u] : 0.f;
+            for (int h = 0; h < 2; h++) {
+                const int r = lane + h * kWave;
                 float dt = 0.f;
 #pragma unroll
                 for (int u = 0; u < 16; u++)
-                    if (k0 + u < i) dt = dt + rv[u] * hv[u];
-                H[(size_t)r * D + i] = (Hr[i] - dt) * inv;
+                    if (u < q) dt = dt + rv[h][u] * hv[u];
+                rv[h][q] = r > i ? (rv[h][q] - dt) * inv : r == i ? dii : rv[h][q];
             }
-            wave_sync();
-            H[(size_t)i * D + i] = dii;
-            wave_sync();
+            pv[q] = low ? rv[0][q] : rv[1][q];
         }
+        uint64_t on[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int r = lane + h * kWave;
+            bool any = false;
+#pragma unroll
+            for (int u = 0; u < 16; u++) {
+                any = any || rv[h][u] != 0.f;
+                if (r >= k0 && r < D && k0 + u <= r && k0 + u < k1) H.at(r, k0 + u) = rv[h][u];
+            }
+            on[h] = wave_ballot(any);
+        }
+        wave_sync();
+        auto empty = [&](int t) { return !(((t < 4 ? on[0] : on[1]) >> (16 * (t & 3))) & 0xffff); };
         for (int Rt = p + 1; Rt < T; Rt++) {
+            if (empty(Rt)) continue;
             for (int Ct = p + 1; Ct <= Rt; Ct++) {
+                if (empty(Ct)) continue;
                 const int ra = Rt * 16 + li, rb = Ct * 16 + li;
                 float a[4], b[4], h[4];
 #pragma unroll
                 for (int kk = 0; kk < 4; kk++) {
                     const int k = k0 + 4 * kk + lk;
-                    a[kk] = (ra < D && k < k1) ? H[(size_t)ra * D + k] : 0.f;
-                    b[kk] = (rb < D && k < k1) ? H[(size_t)rb * D + k] : 0.f;
+                    a[kk] = (ra < D && k < k1) ? H.at(ra, k) : 0.f;
+                    b[kk] = (rb < D && k < k1) ? H.at(rb, k) : 0.f;
                 }
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const int i = Rt * 16 + 4 * lk + r;
-                    h[r] = (i < D && rb <= i) ? H[(size_t)i * D + rb] : 0.f;
+                    h[r] = (i < D && rb <= i) ? H.at(i, rb) : 0.f;
                 }
                 mfma_v4f acc = mfma_v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -526,7 +572,7 @@ __device__ inline void cholesky_blocked_mfma(int D, float* H, float eps, int lan
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const int i = Rt * 16 + 4 * lk + r;
-                    if (i < D && rb <= i) H[(size_t)i * D + rb] = h[r] - acc[r];
+                    if (i < D && rb <= i) H.at(i, rb) = h[r] - acc[r];
                 }
             }
         }
@@ -535,11 +581,13 @@ __device__ inline void cholesky_blocked_mfma(int D, float* H, float eps, int lan
 }
 
 // solver.py:1395-1452 + :1595-1621: H = M + J^T diag(D active) J (lower), then in-place Cholesky
-__device__ inline void wave_hessian_cholesky(const DModel& m, const LState& loc, const WorkRows& R, int lane) {
+template <class HM>
+__device__ __forceinline__ void wave_hessian_cholesky(const DModel& m, const LState& loc, const WorkRows& R, const HM& H,
+                                                      int lane) {
     const int D = m.D;
     if (mfma_model(D)) {
-        wave_hessian_mfma(m, loc, R, lane);
-        cholesky_blocked_mfma(D, FP(loc, nt_H), m.eps, lane);
+        wave_hessian_mfma(m, loc, R, H, lane);
+        cholesky_blocked_mfma(D, H, m.eps, lane);
         return;
     }
     const int nc = LF(n_con, 0);
@@ -582,10 +630,11 @@ __device__ inline void wave_hessian_cholesky(const DModel& m, const LState& loc,
 // lane and lane + 64), a ballot finds the next column it touches (a row touches few; every other column would be a round
 // trip to memory only to find a zero), and that column is loaded while the one before is worked on. Five stacks of four
 // boxes x101: 5.2 M -> 2.5 M cycles a step.
-__device__ inline bool wave_cholesky_incremental(const DModel& m, const LState& loc, const WorkRows& R, int lane) {
+template <class HM>
+__device__ __forceinline__ bool wave_cholesky_incremental(const DModel& m, const LState& loc, const WorkRows& R,
+                                                          const HM& H, int lane) {
     const int D = m.D;
     const int nc = LF(n_con, 0);
-    float* H = FP(loc, nt_H);
     for (int c0 = 0; c0 < nc; c0 += kWave) {
         const int cl = c0 + lane;
         uint64_t flips = wave_ballot(cl < nc && (R.active(cl) ^ R.prev(cl)));
@@ -612,20 +661,20 @@ __device__ inline bool wave_cholesky_incremental(const DModel& m, const LState& 
                     else hi &= hi - 1;
                     const int next = lo ? __builtin_ctzll(lo) : hi ? kWave + __builtin_ctzll(hi) : -1;
                     if (loaded != k) {
-                        dk = H[(size_t)k * D + k];
+                        dk = H.at(k, k);
 #pragma unroll
                         for (int h = 0; h < 2; h++) {
                             const int i = lane + h * kWave;
-                            col[h] = i > k && i < D ? H[(size_t)i * D + k] : 0.f;
+                            col[h] = i > k && i < D ? H.at(i, k) : 0.f;
                         }
                     }
                     float ncol[2] = {0.f, 0.f}, ndk = 0.f;
                     if (next >= 0) {
-                        ndk = H[(size_t)next * D + next];
+                        ndk = H.at(next, next);
 #pragma unroll
                         for (int h = 0; h < 2; h++) {
                             const int i = lane + h * kWave;
-                            ncol[h] = i > next && i < D ? H[(size_t)i * D + next] : 0.f;
+                            ncol[h] = i > next && i < D ? H.at(i, next) : 0.f;
                         }
                     }
                     const float vk = readlane_f(k < kWave ? v[0] : v[1], k & (kWave - 1));
@@ -638,10 +687,10 @@ __device__ inline bool wave_cholesky_incremental(const DModel& m, const LState& 
                         const int i = lane + h * kWave;
                         if (i > k && i < D) {
                             const float x = (col[h] + ss * v[h] * sign) * cinv;
-                            H[(size_t)i * D + k] = x;
+                            H.at(i, k) = x;
                             v[h] = v[h] * cc - ss * x;
                         } else if (i == k) {
-                            H[(size_t)k * D + k] = r;
+                            H.at(k, k) = r;
                         }
                         col[h] = ncol[h];
                     }
@@ -708,10 +757,10 @@ __device__ inline void wave_gradient_cg(const DModel& m, const LState& loc, int 
 // wavefront. Backward substitution column by column: x_i = y_i / L[i][i], then every lane k < i subtracts L[i][k] x_i
 // from its y_k (row i again). The sums run in their own order (a tree forward, descending i backward), as the
 // matrix-core factor already does. Rows are loaded kAhead steps early (the factor may live in global memory).
-__device__ inline void wave_gradient_lanes(const DModel& m, const LState& loc, int lane) {
+template <class HM>
+__device__ __forceinline__ void wave_gradient_lanes(const DModel& m, const LState& loc, const HM& H, int lane) {
     constexpr int kAhead = 4;
     const int D = m.D;
-    const float* L = FP(loc, nt_H);
     float cur[2], hd[2], y[2] = {0.f, 0.f}, x[2] = {0.f, 0.f};
 #pragma unroll
     for (int r = 0; r < 2; r++) {
@@ -722,11 +771,11 @@ __device__ inline void wave_gradient_lanes(const DModel& m, const LState& loc, i
             const float g = LF(Ma, i) - LF(force, i) - LF(qfrc_constraint, i);
             LF(grad, i) = g;
             cur[r] = g;
-            hd[r] = L[i * D + i];
+            hd[r] = H.at(i, i);
         }
     }
     // L[i][k] for k < i (row i, strictly below the diagonal), else 0
-    auto rowv = [&](int i, int k) { return (i >= 0 && i < D && k < i) ? L[i * D + k] : 0.f; };
+    auto rowv = [&](int i, int k) { return (i >= 0 && i < D && k < i) ? H.at(i, k) : 0.f; };
     float pf[kAhead][2];
 #pragma unroll
     for (int k = 0; k < kAhead; k++)
@@ -1453,9 +1502,10 @@ __device__ inline void export_row_forces(const DModel& m, const LState& loc, con
 
 // solver.py:2936-3059 (init), :3063-3139 (Newton or conjugate-gradient iteration), :3164-3190 (body), :3241-3261,
 // :3199-3237
-template <int KD>
+// H: the factor of the models with 25 to 128 dofs (KD = 0); every other model keeps its own in nt_H.
+template <int KD, class HM>
 __device__ inline void wave_solve(const DModel& m, const LState& loc, const DState& st, int b, const WorkRows& R,
-                                  int lane, float* tile) {
+                                  int lane, float* tile, const HM& H) {
     const int D = m.D;
     const int nc = LF(n_con, 0);
     const bool ws = nc > 0 && LF(is_warmstart, 0);
@@ -1471,7 +1521,16 @@ __device__ inline void wave_solve(const DModel& m, const LState& loc, const DSta
         LF(Ma, d1) = ma;
     }
     for (int c = lane; c < nc; c += kWave) {
-        R.Jaref(c) = seq_sum(-R.aref(c), 0, D, [&](int d) { return R.jac(c, d) * LF(qacc, d); });
+        if (lane_dofs) {  // the tiles that are all zero add nothing
+            float ja = -R.aref(c);
+            for (int on = R.tiles(c); on; on &= on - 1) {
+                const int d0 = 16 * __builtin_ctz(on);
+                ja = seq_sum(ja, d0, min(d0 + 16, D), [&](int d) { return R.jac(c, d) * LF(qacc, d); });
+            }
+            R.Jaref(c) = ja;
+        } else {
+            R.Jaref(c) = seq_sum(-R.aref(c), 0, D, [&](int d) { return R.jac(c, d) * LF(qacc, d); });
+        }
         R.active(c) = 0;  // the first update compares against a cleared previous active set
     }
     wave_sync();
@@ -1485,9 +1544,9 @@ __device__ inline void wave_solve(const DModel& m, const LState& loc, const DSta
         wave_gradient_cg(m, loc, lane);
     } else {
         if constexpr (KD > 0) wave_hessian_cholesky_tiled<KD>(m, loc, R, lane, tile);
-        else wave_hessian_cholesky(m, loc, R, lane);
+        else wave_hessian_cholesky(m, loc, R, H, lane);
         if constexpr (KD > 0) wave_gradient_r<KD>(m, loc, lane);
-        else if (D <= 2 * kWave) wave_gradient_lanes(m, loc, lane);
+        else if (D <= 2 * kWave) wave_gradient_lanes(m, loc, H, lane);
         else wave_gradient(m, loc);
     }
     if (lane_dofs) {
@@ -1525,13 +1584,13 @@ __device__ inline void wave_solve(const DModel& m, const LState& loc, const DSta
                 } else {
                     bool degenerate;
                     if constexpr (KD > 0) degenerate = wave_cholesky_incremental_r<KD>(m, loc, R, lane, tile);
-                    else degenerate = wave_cholesky_incremental(m, loc, R, lane);
+                    else degenerate = wave_cholesky_incremental(m, loc, R, H, lane);
                     if (degenerate) {
                         if constexpr (KD > 0) wave_hessian_cholesky_tiled<KD>(m, loc, R, lane, tile);
-                        else wave_hessian_cholesky(m, loc, R, lane);
+                        else wave_hessian_cholesky(m, loc, R, H, lane);
                     }
                     if constexpr (KD > 0) wave_gradient_r<KD>(m, loc, lane);
-                    else if (D <= 2 * kWave) wave_gradient_lanes(m, loc, lane);
+                    else if (D <= 2 * kWave) wave_gradient_lanes(m, loc, H, lane);
                     else wave_gradient(m, loc);
                 }
                 float gn = 0.f;
