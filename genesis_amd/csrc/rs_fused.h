@@ -365,10 +365,10 @@ __device__ inline void wave_integrate(const DModel& m, const LState& loc, int la
 
 // One environment's substep on the calling wavefront (w = wavefront index in the workgroup).
 // kPath: 1 = models in the first row-tile class (at most kTileMaxDofs dofs), 4 = the second (up to kTileWideDofs),
-// 5 = larger models with short constraint rows (island solver), 0 = the others, 2 = any (decided per call: the shared
-// launch of several models). Returns the narrowphase's GJK/EPA
-// work (see wave_narrowphase).
-template <bool kLds, int kPath = 2>
+// 5 = larger models with short constraint rows (island solver), 0 = the others; decided per call (the shared launch of
+// several models): 2 = any, 6 = models of up to kTileWideDofs. Returns the narrowphase's GJK/EPA work (see
+// wave_narrowphase).
+template <bool kLds, int kPath>
 __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, const FusedArgs& fa,
                                           const RS_CONST int* loc_off, int b, int w, float* lds_env) {
     const int lane = lane_id();
@@ -392,7 +392,7 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
     if constexpr (kPath == 1 || kPath == 4)
         if (FP(loc, n_con)[0] >= kSchedHeavyRows) __builtin_amdgcn_s_setprio(3);
     // kernel_step_1: CRBA, L^T D L, actuation + passive + bias forces, acc_smooth
-    constexpr bool kMany = kPath != 1 && kPath != 4;
+    constexpr bool kMany = kPath != 1 && kPath != 4 && kPath != 6;
     wave_mass_matrix<kMany>(m, loc, lane);
     wave_factor_mass(m, loc, lane);
     wave_torque_passive(m, loc, lane);
@@ -418,8 +418,8 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
             Q = row_groups(m, wk, fa);
             island_constraints(m, loc, st, b, R, Q, lane, tile);
         } else {
-            wave_constraints(m, loc, st, b, R, lane, tile, kPath == 1 || kPath == 4 || (kPath == 2 && fa.tiled != 0),
-                             fa.row_width);
+            const bool tiled = kPath == 1 || kPath == 4 || kPath == 6 || (kPath == 2 && fa.tiled != 0);
+            wave_constraints(m, loc, st, b, R, lane, tile, tiled, fa.row_width);
         }
         const SquareH square{FP(loc, nt_H), m.D};
         if constexpr (kPath == 5) {
@@ -430,10 +430,14 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
         else if constexpr (kPath == 0) {
             if (fa.h_off >= 0) wave_solve<0>(m, loc, st, b, R, lane, tile, PackedH{slice + fa.h_off});
             else wave_solve<0>(m, loc, st, b, R, lane, tile, square);
-        } else if (islands) island_solve<false>(m, loc, st, b, R, Q, lane, tile, triangles_in_record(loc));
-        else if (fa.tiled == kTileMaxDofs) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile, square);
-        else if (fa.tiled == kTileWideDofs) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile, square);
-        else wave_solve<0>(m, loc, st, b, R, lane, tile, square);
+        } else if (fa.tiled == kTileMaxDofs) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile, square);
+        else if (kPath == 6 || fa.tiled == kTileWideDofs) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile, square);
+        else if constexpr (kPath == 2) {
+            if (islands && fa.h_off >= 0) island_solve<true>(m, loc, st, b, R, Q, lane, tile, slice + fa.h_off);
+            else if (islands) island_solve<false>(m, loc, st, b, R, Q, lane, tile, triangles_in_record(loc));
+            else if (fa.h_off >= 0) wave_solve<0>(m, loc, st, b, R, lane, tile, PackedH{slice + fa.h_off});
+            else wave_solve<0>(m, loc, st, b, R, lane, tile, square);
+        }
     }
     // kernel_step_2: cacc, semi-implicit Euler, forward kinematics and velocities
     wave_update_acc<kMany>(m, loc, lane, true);
@@ -538,20 +542,26 @@ struct FusedSegment {
 
 // Several models and slabs in one launch (the serving loop's co-batched step). Every segment uses the launch's
 // environments-per-workgroup; a workgroup finds its segment by scanning the table (a few dozen entries at most).
-template <bool kLds>
-__global__ void __launch_bounds__(512) k_fused_multi(const FusedSegment* __restrict__ segs, int n_segs) {
+// kPath 6: every model has a row tile. kPath 2: some model has more than 24 dofs; its environments are the longest, so
+// the launch gives every wavefront all registers of its SIMD and room for the Hessian in LDS, and keeps the private
+// regions in memory (1000 quadrupeds, 333 arms and 100 piles: 10.9 -> 10.3 ms for 4 ticks, against two wavefronts per
+// SIMD; 8 piles with 16384 quadrupeds, which would rather have the second wavefront, 21.8 -> 23.9 ms).
+template <bool kLds, int kPath>
+__global__ void __launch_bounds__(kPath == 2 ? kWave : 512)
+k_fused_multi(const FusedSegment* __restrict__ segs, int n_segs) {
     extern __shared__ float lds_env[];
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
-    // the table does not change while the kernel runs: read through the constant address space, its entries (the model's
-    // and the slab's pointers among them) are scalar loads
-    const FusedSegment* tab = (const FusedSegment*)(const RS_CONST FusedSegment*)(uintptr_t)segs;
+    // The table does not change while the kernel runs: read through the constant address space, its entries (the model's
+    // and the slab's pointers among them) are scalar loads.
+    const FusedSegment* tab = segs;
+    if constexpr (kPath == 2) tab = (const FusedSegment*)(const RS_CONST FusedSegment*)(uintptr_t)segs;
     int s = 0;
     while (s + 1 < n_segs && tab[s + 1].first_block <= blk) s++;
     const FusedSegment& g = tab[s];
     const int b = (blk - g.first_block) * g.fa.epb + w;
     if (b >= g.st.B) return;
-    fused_env<kLds>(g.m, g.st, g.fa, (const RS_CONST int*)g.fa.loc_off, b, w, lds_env);
+    fused_env<kLds, kPath>(g.m, g.st, g.fa, (const RS_CONST int*)g.fa.loc_off, b, w, lds_env);
 }
 
 }  // namespace rs

@@ -20,7 +20,7 @@ void launch_fused_island(bool use_lds, dim3 grid, dim3 block, size_t lds_bytes, 
 void launch_fused_generic(bool use_lds, dim3 grid, dim3 block, size_t lds_bytes, hipStream_t s, const DModel& m,
                           const DState& st, const FusedArgs& fa);
 // k_fused_multi: one fused substep of several (model, slab) segments
-void launch_fused_multi(bool use_lds, dim3 grid, dim3 block, size_t lds_bytes, hipStream_t s,
+void launch_fused_multi(bool use_lds, bool large, dim3 grid, dim3 block, size_t lds_bytes, hipStream_t s,
                         const FusedSegment* segs, int n_segs);
 
 }  // namespace rs

@@ -90,12 +90,11 @@ static int64_t work_floats(const rs_model_header& h, int row_width);
 
 // Whether a model with short rows takes the island solver. Its results differ from the dense solver's in the last bits,
 // as those of any two orders of summing do, and a contact that a detection finds or misses by a last bit moves its
-// environment visibly. MPR's perturbed box-box detections have such edges all the time (a resting pile of 20 boxes: one
-// environment in 200 within four steps), so models with them keep the dense solver's sums, bit for bit, at 2.3 times the
-// island solver's time. The separating-axis test meets one in 7000 environments of stacked boxes within four steps and
-// none in 14000 of a resting pile; models with no collision pairs have none.
+// environment visibly: MPR's perturbed box-box detections do so in one environment of 200 within four steps (a resting
+// pile of 20 boxes), the separating-axis test in one of 7000 (stacked boxes). Models with collision pairs therefore keep
+// the dense solver's sums, bit for bit, at 2.3 times the island solver's time; the others have no such edge.
 static bool takes_islands(const rs_model_header& h, int row_width) {
-    return row_width > 0 && (h.box_box_detection || !h.enable_collision || h.n_pairs == 0);
+    return row_width > 0 && (!h.enable_collision || h.n_pairs == 0);
 }
 
 // row_width: the model's row width (RS_N_WORK depends on it)
@@ -193,10 +192,10 @@ static int lds_slice_floats(const rs_model_header& h, const FusedArgs& fa, bool 
 }
 // the packed lower triangle of the Hessian of models above 24 dofs follows in the slice when the workgroup's slices still
 // fit with it (it is in nt_H otherwise): every step of a factorisation or a triangular solve waits for a round trip to it
-static int slice_with_triangles(const rs_model* m, const FusedArgs& fa, bool use_lds, int* h_off) {
+static int slice_with_triangles(const rs_model* m, const FusedArgs& fa, bool use_lds, int* h_off, int max_lds) {
     const int slice = lds_slice_floats(m->h, fa, use_lds), with_h = slice + tri4(m->h.n_dofs);
     const bool wanted = fa.islands || (!fa.tiled && !use_lds && m->h.n_dofs <= kMfmaMaxDofs);
-    const bool in_lds = wanted && (int64_t)fa.epb * with_h * 4 <= m->max_lds;
+    const bool in_lds = wanted && (int64_t)fa.epb * with_h * 4 <= max_lds;
     *h_off = in_lds ? slice : -1;
     return in_lds ? with_h : slice;
 }
@@ -487,7 +486,7 @@ static int fused_substep(const rs_model* m, const DState& st, hipStream_t s) {
     if (fa.sched) hipLaunchKernelGGL(k_sched_flip, dim3(1), dim3(1), 0, s, st);
     const dim3 grid((unsigned)((st.B + epb - 1) / epb)), block((unsigned)(kWave * epb));
     int h_off = -1;
-    set_lds_slice(m->h, &fa, m->use_lds, slice_with_triangles(m, fa, m->use_lds, &h_off));
+    set_lds_slice(m->h, &fa, m->use_lds, slice_with_triangles(m, fa, m->use_lds, &h_off, m->max_lds));
     fa.h_off = h_off;
     const size_t lds = (size_t)epb * fa.lds_wave * 4;
     // one kernel variant per (private region, occupancy) for models with a row tile; models without one run the
@@ -680,7 +679,7 @@ int rs_fused_config_get(const rs_model* m, rs_fused_config* out) {
     out->envs_per_block = m->fa.epb;
     out->use_lds = m->use_lds;
     int h_off;
-    out->lds_bytes_per_env = slice_with_triangles(m, m->fa, m->use_lds, &h_off) * 4;
+    out->lds_bytes_per_env = slice_with_triangles(m, m->fa, m->use_lds, &h_off, m->max_lds) * 4;
     out->schedule = m->schedule;
     out->occupancy = m->occupancy;
     out->gjk_lds = m->fa.gjk_words > 0;
@@ -937,17 +936,17 @@ int rs_batch_step(rs_batch* bt, int n, const rs_model* const* models, void* cons
     if (!bt || n < 1 || n > bt->max_segments || !models || !states || !n_envs)
         return fail(RS_E_INVALID, "rs_batch_step: bad argument");
     hipStream_t s = (hipStream_t)stream;
-    const int epb = 2;
-    int slice_lds = 0, slice_hbm = 0;
+    int epb = 2, slice_lds = 0, slice = 0;
+    bool large = false;
     for (int i = 0; i < n; i++) {
         if (!models[i] || !states[i] || n_envs[i] < 1) return fail(RS_E_INVALID, "rs_batch_step: bad segment");
         slice_lds = std::max(slice_lds, lds_slice_floats(models[i]->h, models[i]->fa, true));
-        slice_hbm = std::max(slice_hbm, lds_slice_floats(models[i]->h, models[i]->fa, false));
+        large = large || !models[i]->fa.tiled;
     }
     int max_lds = models[0]->max_lds;
     for (int i = 1; i < n; i++) max_lds = max_lds < models[i]->max_lds ? max_lds : models[i]->max_lds;
-    const bool use_lds = (int64_t)epb * slice_lds * 4 <= max_lds;
-    const int slice = use_lds ? slice_lds : slice_hbm;
+    const bool use_lds = !large && (int64_t)epb * slice_lds * 4 <= max_lds;
+    if (large) epb = 1;
     const int k = bt->slot;
     bt->slot = (bt->slot + 1) % rs_batch::kRing;
     if (bt->pending[k]) HIP_OK(hipEventSynchronize(bt->done[k]));
@@ -957,18 +956,23 @@ int rs_batch_step(rs_batch* bt, int n, const rs_model* const* models, void* cons
         tab[i].m = models[i]->dm;
         tab[i].st = make_state(models[i], states[i], n_envs[i]);
         tab[i].fa = models[i]->fa;
-        set_lds_slice(models[i]->h, &tab[i].fa, use_lds, slice);
         tab[i].fa.epb = epb;
+        int h_off = -1;
+        const int own = use_lds ? slice_lds : slice_with_triangles(models[i], tab[i].fa, false, &h_off, max_lds);
+        set_lds_slice(models[i]->h, &tab[i].fa, use_lds, own);
+        tab[i].fa.h_off = h_off;
+        slice = std::max(slice, own);
         tab[i].fa.sched = 0;
         tab[i].first_block = blocks;
         tab[i].n_blocks = (n_envs[i] + epb - 1) / epb;
         blocks += tab[i].n_blocks;
     }
+    for (int i = 0; i < n; i++) tab[i].fa.lds_wave = slice;
     HIP_OK(hipMemcpyAsync(bt->dev[k], tab, sizeof(FusedSegment) * n, hipMemcpyHostToDevice, s));
     HIP_OK(hipEventRecord(bt->done[k], s));
     bt->pending[k] = true;
     const dim3 grid((unsigned)blocks), block((unsigned)(kWave * epb));
-    launch_fused_multi(use_lds, grid, block, (size_t)epb * slice * 4, s, bt->dev[k], n);
+    launch_fused_multi(use_lds, large, grid, block, (size_t)epb * slice * 4, s, bt->dev[k], n);
     HIP_OK(hipGetLastError());
     return RS_OK;
 }
