@@ -545,7 +545,7 @@ struct FusedSegment {
 // kPath 6: every model has a row tile. kPath 2: some model has more than 24 dofs; its environments are the longest, so
 // the launch gives every wavefront all registers of its SIMD and room for the Hessian in LDS, and keeps the private
 // regions in memory (1000 quadrupeds, 333 arms and 100 piles: 10.9 -> 10.3 ms for 4 ticks, against two wavefronts per
-// SIMD; 8 piles with 16384 quadrupeds, which would rather have the second wavefront, 21.8 -> 23.9 ms).
+// SIMD; 8 piles with 16384 quadrupeds, which would rather have the second wavefront, 21.8 -> 22.9 ms).
 template <bool kLds, int kPath>
 __global__ void __launch_bounds__(kPath == 2 ? kWave : 512)
 k_fused_multi(const FusedSegment* __restrict__ segs, int n_segs) {
