@@ -6,7 +6,6 @@
 #include "rs_collision.h"
 #include "rs_constraint.h"
 #include "rs_dyn.h"
-#include "rs_island_solver.h"
 #include "rs_wave.h"
 #include "rs_wave_dyn.h"
 #include "rs_wave_solver.h"
@@ -365,7 +364,7 @@ __device__ inline void wave_integrate(const DModel& m, const LState& loc, int la
 
 // One environment's substep on the calling wavefront (w = wavefront index in the workgroup).
 // kPath: 1 = models in the first row-tile class (at most kTileMaxDofs dofs), 4 = the second (up to kTileWideDofs),
-// 5 = larger models with short constraint rows (island solver), 0 = the others; decided per call (the shared launch of
+// 0 = larger models; decided per call (the shared launch of
 // several models): 2 = any, 6 = models of up to kTileWideDofs. Returns the narrowphase's GJK/EPA work (see
 // wave_narrowphase).
 template <bool kLds, int kPath>
@@ -381,8 +380,7 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
     float* base = kLds ? slice : in_place ? (float*)((uint32_t*)(void*)st.qpos + (size_t)b * st.LS) : wk + fa.off_loc;
     float* tile = slice + fa.tile_off;
     const LState loc = make_local(base, loc_off);
-    const bool islands = kPath == 5 || (kPath == 2 && fa.islands);
-    const WorkRows R{wk + fa.off_jac, wk + fa.off_rowf, wk + fa.off_tmp, m.CMAX, islands ? fa.row_width : m.D};
+    const WorkRows R{wk + fa.off_jac, wk + fa.off_rowf, wk + fa.off_tmp, m.CMAX, m.D};
 
     if (!in_place) stage_local<true>(st, (uint32_t*)base, fa.n_local, b, lane);
     wave_sync();
@@ -413,19 +411,10 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
     }
     // ConstraintSolver.resolve
     if (!m.disable_constraint) {
-        RowGroups Q;
-        if (islands) {
-            Q = row_groups(m, wk, fa);
-            island_constraints(m, loc, st, b, R, Q, lane, tile);
-        } else {
-            const bool tiled = kPath == 1 || kPath == 4 || kPath == 6 || (kPath == 2 && fa.tiled != 0);
-            wave_constraints(m, loc, st, b, R, lane, tile, tiled, fa.row_width);
-        }
+        const bool tiled = kPath == 1 || kPath == 4 || kPath == 6 || (kPath == 2 && fa.tiled != 0);
+        wave_constraints(m, loc, st, b, R, lane, tile, tiled, fa.row_width);
         const SquareH square{FP(loc, nt_H), m.D};
-        if constexpr (kPath == 5) {
-            if (fa.h_off >= 0) island_solve<true>(m, loc, st, b, R, Q, lane, tile, slice + fa.h_off);
-            else island_solve<false>(m, loc, st, b, R, Q, lane, tile, triangles_in_record(loc));
-        } else if constexpr (kPath == 1) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile, square);
+        if constexpr (kPath == 1) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile, square);
         else if constexpr (kPath == 4) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile, square);
         else if constexpr (kPath == 0) {
             if (fa.h_off >= 0) wave_solve<0>(m, loc, st, b, R, lane, tile, PackedH{slice + fa.h_off});
@@ -433,9 +422,7 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
         } else if (fa.tiled == kTileMaxDofs) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile, square);
         else if (kPath == 6 || fa.tiled == kTileWideDofs) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile, square);
         else if constexpr (kPath == 2) {
-            if (islands && fa.h_off >= 0) island_solve<true>(m, loc, st, b, R, Q, lane, tile, slice + fa.h_off);
-            else if (islands) island_solve<false>(m, loc, st, b, R, Q, lane, tile, triangles_in_record(loc));
-            else if (fa.h_off >= 0) wave_solve<0>(m, loc, st, b, R, lane, tile, PackedH{slice + fa.h_off});
+            if (fa.h_off >= 0) wave_solve<0>(m, loc, st, b, R, lane, tile, PackedH{slice + fa.h_off});
             else wave_solve<0>(m, loc, st, b, R, lane, tile, square);
         }
     }
@@ -524,7 +511,7 @@ k_fused_wave(DModel m, DState st, FusedArgs fa) {
     fused_launch<kLds, kPath>(m, st, fa, (const RS_CONST int*)fa.loc_off);
 }
 
-// Models above 24 dofs (kPath 5 and 0): at most kGenericMaxThreads lanes (4 environments) per workgroup, so that a
+// Models above 24 dofs (kPath 0): at most kGenericMaxThreads lanes (4 environments) per workgroup, so that a
 // wavefront may hold all 512 registers of its SIMD.
 template <bool kLds, int kPath>
 __global__ void __launch_bounds__(kGenericMaxThreads) k_fused_large(FusedKernArgs) {

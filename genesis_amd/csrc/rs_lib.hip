@@ -86,19 +86,10 @@ struct rs_graph {
     hipGraphExec_t exec = nullptr;
 };
 
-static int64_t work_floats(const rs_model_header& h, int row_width);
+static int64_t work_floats(const rs_model_header& h);
+static int64_t field_rows(const rs_model_header& h, int i);
 
-// Whether a model with short rows takes the island solver. Its results differ from the dense solver's in the last bits,
-// as those of any two orders of summing do, and a contact that a detection finds or misses by a last bit moves its
-// environment visibly: MPR's perturbed box-box detections do so in one environment of 200 within four steps (a resting
-// pile of 20 boxes), the separating-axis test in one of 7000 (stacked boxes). Models with collision pairs therefore keep
-// the dense solver's sums, bit for bit, at 2.3 times the island solver's time; the others have no such edge.
-static bool takes_islands(const rs_model_header& h, int row_width) {
-    return row_width > 0 && (!h.enable_collision || h.n_pairs == 0);
-}
-
-// row_width: the model's row width (RS_N_WORK depends on it)
-static int64_t count_of(const rs_model_header& h, int kind, int row_width = 0) {
+static int64_t count_of(const rs_model_header& h, int kind) {
     switch (kind) {
         case RS_N_ONE: return 1;
         case RS_N_LINKS: return h.n_links;
@@ -118,7 +109,7 @@ static int64_t count_of(const rs_model_header& h, int kind, int row_width = 0) {
         case RS_N_CONSTRAINTS_DOFS: return (int64_t)h.len_constraints * h.n_dofs;
         case RS_N_BROAD: return h.max_collision_pairs_broad;
         case RS_N_SORT: return 2 * (int64_t)h.n_geoms;
-        case RS_N_WORK: return work_floats(h, row_width);
+        case RS_N_WORK: return work_floats(h);
         case RS_N_SCHED: return sched_rows();
         case RS_N_DOFS_PLANE: return h.n_dofs;
         case RS_N_ONE_PLANE: return 1;
@@ -127,14 +118,14 @@ static int64_t count_of(const rs_model_header& h, int kind, int row_width = 0) {
 }
 
 // rows per environment of state field i (at least 1, so that every plane is addressable even for empty models)
-static int64_t field_rows(const rs_model_header& h, int i, int row_width = 0) {
-    int64_t rows = count_of(h, k_state_fields[i].count, row_width) * k_state_fields[i].width;
+static int64_t field_rows(const rs_model_header& h, int i) {
+    int64_t rows = count_of(h, k_state_fields[i].count) * k_state_fields[i].width;
     return rows < 1 ? 1 : rows;
 }
 
 // Private-region offsets of the local fields and the env-major work layout of the fused kernel (floats, each
 // sub-array 16-byte aligned, each environment's slice 256-byte aligned).
-static void fused_layout(const rs_model_header& h, FusedArgs* fa, int row_width) {
+static void fused_layout(const rs_model_header& h, FusedArgs* fa) {
     auto up4 = [](int64_t x) { return (x + 3) / 4 * 4; };
     // local fields come first in the directory; the private region mirrors their packed planes row for row
     int64_t off = 0;
@@ -153,19 +144,12 @@ static void fused_layout(const rs_model_header& h, FusedArgs* fa, int row_width)
     fa->gjk_off = -1;
     fa->lds_wave = (int)up4((int64_t)kTileStride * tile_rows(h.n_dofs));
     fa->sched = 0;
-    fa->row_width = row_width;
-    fa->islands = takes_islands(h, row_width);
+    fa->row_width = 0;
     fa->h_off = -1;
     const int64_t C = h.len_constraints > 0 ? h.len_constraints : 1, D = h.n_dofs;
     fa->off_loc = 0;
     fa->off_jac = (int)up4(off);
-    // the jacobian rows: dense, or the island solver's row groups (rs_island_solver.h row_groups)
-    int64_t jac = up4(C * D);
-    if (fa->islands) {
-        const int64_t G = row_group_max(h.n_equalities, h.n_dofs, h.max_contact_pairs);
-        jac = std::max(jac, up4(C * row_width + G * (row_width / 4 + 5 + D) + (6 * (int64_t)h.n_equalities + D) * D));
-    }
-    fa->off_rowf = (int)(fa->off_jac + jac);
+    fa->off_rowf = (int)(fa->off_jac + up4(C * D));
     fa->off_tmp = (int)(fa->off_rowf + RW_COUNT * up4(C));
     fa->off_pc = (int)(fa->off_tmp + kTmpArrays * up4(C));
     fa->off_mc = (int)(fa->off_pc + up4((int64_t)kWave * (h.n_contacts_per_pair > 0 ? h.n_contacts_per_pair : 1) * 8));
@@ -178,10 +162,10 @@ static void fused_layout(const rs_model_header& h, FusedArgs* fa, int row_width)
 // LDS slice of one wavefront: the private region (when it is in LDS) followed by the row tile (models with short rows: the
 // tile rows that stage one and four words per link)
 static int tile_floats(const rs_model_header& h, const FusedArgs& fa) {
-    if (fa.row_width > 0) return kTileStride * island_tile_rows(fa.row_width) + 4 * h.n_links;
+    if (fa.row_width > 0) return kTileStride * short_row_tile_rows(fa.row_width) + 4 * h.n_links;
     return (kTileStride * tile_rows(h.n_dofs) + 3) / 4 * 4;
 }
-// slice layout: [private region (LDS mode)][row tile][GJK/EPA polytope (models with mesh geoms)][island triangles]
+// slice layout: [private region (LDS mode)][row tile][GJK/EPA polytope (models with mesh geoms)][packed Hessian]
 static void set_lds_slice(const rs_model_header& h, FusedArgs* fa, bool use_lds, int slice_floats) {
     fa->tile_off = use_lds ? fa->loc_floats : 0;
     fa->gjk_off = fa->gjk_words > 0 ? fa->tile_off + tile_floats(h, *fa) : -1;
@@ -192,17 +176,17 @@ static int lds_slice_floats(const rs_model_header& h, const FusedArgs& fa, bool 
 }
 // the packed lower triangle of the Hessian of models above 24 dofs follows in the slice when the workgroup's slices still
 // fit with it (it is in nt_H otherwise): every step of a factorisation or a triangular solve waits for a round trip to it
-static int slice_with_triangles(const rs_model* m, const FusedArgs& fa, bool use_lds, int* h_off, int max_lds) {
+static int slice_with_hessian(const rs_model* m, const FusedArgs& fa, bool use_lds, int* h_off, int max_lds) {
     const int slice = lds_slice_floats(m->h, fa, use_lds), with_h = slice + tri4(m->h.n_dofs);
-    const bool wanted = fa.islands || (!fa.tiled && !use_lds && m->h.n_dofs <= kMfmaMaxDofs);
+    const bool wanted = !fa.tiled && !use_lds && m->h.n_dofs <= kMfmaMaxDofs;
     const bool in_lds = wanted && (int64_t)fa.epb * with_h * 4 <= max_lds;
     *h_off = in_lds ? slice : -1;
     return in_lds ? with_h : slice;
 }
 
-static int64_t work_floats(const rs_model_header& h, int row_width) {
+static int64_t work_floats(const rs_model_header& h) {
     FusedArgs fa;
-    fused_layout(h, &fa, row_width);
+    fused_layout(h, &fa);
     return fa.work_stride;
 }
 
@@ -226,7 +210,7 @@ static void layout(const rs_model* m, int n_envs, int64_t* offs, int64_t* total)
     const int64_t rec = record_floats(m);
     int64_t off = 0, in_rec = 0;
     for (int i = 0; i < k_n_state_fields; i++) {
-        const int64_t rows = field_rows(m->h, i, m->fa.row_width);
+        const int64_t rows = field_rows(m->h, i);
         const bool local = is_local_kind(k_state_fields[i].count);
         if (local && rec > 0) {
             offs[i] = in_rec * 4;
@@ -486,16 +470,15 @@ static int fused_substep(const rs_model* m, const DState& st, hipStream_t s) {
     if (fa.sched) hipLaunchKernelGGL(k_sched_flip, dim3(1), dim3(1), 0, s, st);
     const dim3 grid((unsigned)((st.B + epb - 1) / epb)), block((unsigned)(kWave * epb));
     int h_off = -1;
-    set_lds_slice(m->h, &fa, m->use_lds, slice_with_triangles(m, fa, m->use_lds, &h_off, m->max_lds));
+    set_lds_slice(m->h, &fa, m->use_lds, slice_with_hessian(m, fa, m->use_lds, &h_off, m->max_lds));
     fa.h_off = h_off;
     const size_t lds = (size_t)epb * fa.lds_wave * 4;
     // one kernel variant per (private region, occupancy) for models with a row tile; models without one run the
     // generic-solver variants at the compiler's register budget (each class is instantiated in its own translation
-    // unit: rs_fused_t16.hip, rs_fused_t24.hip, rs_fused_island.hip, rs_fused_gen.hip)
+    // unit: rs_fused_t16.hip, rs_fused_t24.hip, rs_fused_gen.hip)
     const bool lds_on = m->use_lds != 0;
     if (fa.tiled == kTileMaxDofs) launch_fused_tile16(lds_on, m->occupancy, grid, block, lds, s, m->dm, st, fa);
     else if (fa.tiled == kTileWideDofs) launch_fused_tile24(lds_on, m->occupancy, grid, block, lds, s, m->dm, st, fa);
-    else if (fa.islands) launch_fused_island(lds_on, grid, block, lds, s, m->dm, st, fa);
     else launch_fused_generic(lds_on, grid, block, lds, s, m->dm, st, fa);
     HIP_OK(hipGetLastError());
     return RS_OK;
@@ -568,8 +551,8 @@ static bool has_convex_mesh(const rs_model_header& h, const char* blob) {
 // of the longest chain of links (two for a row between joints). 0 for models that the row-tile solvers serve, with
 // more dofs than two per lane, or whose rows are longer than kRowWidthMax (a long chain: its rows are better taken as
 // dense, on the matrix cores).
-static int island_row_width(const rs_model_header& h, const char* blob) {
-    if (h.n_dofs <= kTileWideDofs || h.n_dofs > kIslandMaxDofs) return 0;
+static int short_row_width(const rs_model_header& h, const char* blob) {
+    if (h.n_dofs <= kTileWideDofs || h.n_dofs > kMfmaMaxDofs) return 0;
     const int32_t *parent = nullptr, *d0 = nullptr, *d1 = nullptr;
     for (int i = 0; i < k_n_model_arrays; i++) {
         const int32_t* a = (const int32_t*)(blob + h.array_offset[i]);
@@ -642,7 +625,8 @@ int rs_model_create(const rs_model_header* h, const void* blob, size_t blob_byte
         return fail(RS_E_INVALID, "rs_model_create: integrator must be one of RS_INTEGRATOR_*");
     }
     static_assert(k_n_state_fields <= kMaxStateFields, "FusedArgs::loc_off too small");
-    fused_layout(m->h, &m->fa, island_row_width(*h, (const char*)blob));
+    fused_layout(m->h, &m->fa);
+    m->fa.row_width = short_row_width(*h, (const char*)blob);
     d.work_stride = m->fa.work_stride;
     d.off_gjk = m->fa.off_gjk;
     // models with convex mesh geoms meet the GJK/EPA hand-over often (deep overlaps of hulls): their wavefronts may
@@ -679,7 +663,7 @@ int rs_fused_config_get(const rs_model* m, rs_fused_config* out) {
     out->envs_per_block = m->fa.epb;
     out->use_lds = m->use_lds;
     int h_off;
-    out->lds_bytes_per_env = slice_with_triangles(m, m->fa, m->use_lds, &h_off, m->max_lds) * 4;
+    out->lds_bytes_per_env = slice_with_hessian(m, m->fa, m->use_lds, &h_off, m->max_lds) * 4;
     out->schedule = m->schedule;
     out->occupancy = m->occupancy;
     out->gjk_lds = m->fa.gjk_words > 0;
@@ -707,7 +691,7 @@ int rs_fused_config_set(rs_model* m, const rs_fused_config* c) {
 
 int rs_state_field_rows(const rs_model* m, int i, int64_t* rows) {
     if (!m || !rows || i < 0 || i >= k_n_state_fields) return fail(RS_E_INVALID, "rs_state_field_rows: bad argument");
-    *rows = field_rows(m->h, i, m->fa.row_width);
+    *rows = field_rows(m->h, i);
     return RS_OK;
 }
 
@@ -958,7 +942,7 @@ int rs_batch_step(rs_batch* bt, int n, const rs_model* const* models, void* cons
         tab[i].fa = models[i]->fa;
         tab[i].fa.epb = epb;
         int h_off = -1;
-        const int own = use_lds ? slice_lds : slice_with_triangles(models[i], tab[i].fa, false, &h_off, max_lds);
+        const int own = use_lds ? slice_lds : slice_with_hessian(models[i], tab[i].fa, false, &h_off, max_lds);
         set_lds_slice(models[i]->h, &tab[i].fa, use_lds, own);
         tab[i].fa.h_off = h_off;
         slice = std::max(slice, own);

@@ -30,7 +30,6 @@ struct FusedArgs {
     int gjk_off;       // offset of that polytope in the wavefront's LDS slice (-1: none)
     int tile_off;      // offset of the row tile (kTileStride x tile_rows(D) floats) in the wavefront's LDS slice
     int row_width;     // most dofs a constraint row touches, a multiple of 4 (models with 25 to 128 dofs; 0: over 32)
-    int islands;       // 1: the island solver (rs_island_solver.h)
     int h_off;         // offset of the packed Hessian of models above 24 dofs in the wavefront's LDS slice (-1: in nt_H)
     int sched;         // 1: map wavefronts to environments through the cost-ordered queues
     int loc_off[kMaxStateFields];  // private-region offset of each state field (local kinds only)
@@ -52,18 +51,12 @@ __host__ __device__ constexpr int tile_class(int n_dofs) {
     return n_dofs <= kTileMaxDofs ? kTileMaxDofs : n_dofs <= kTileWideDofs ? kTileWideDofs : 0;
 }
 
-// Island solver (models with 25 to 128 dofs whose rows touch at most kRowWidthMax of them): row width (a multiple of
-// 4), tile rows that stage the contact rows, words of LDS its island search needs (at most a tile), groups of rows, and
-// the words of a packed lower triangle of n rows, every row padded to a multiple of 4 so that rows are 16-byte aligned
-// (tri4(i) is also the offset of row i).
-constexpr int kIslandMaxDofs = 2 * kWave;
+// Models with 25 to 128 dofs whose rows touch at most kRowWidthMax of them: rows of the tile that stages their contact
+// rows; and the words of a packed lower triangle of n rows, every row padded to a multiple of 4 so that rows are 16-byte
+// aligned (tri4(i) is also the offset of row i).
 constexpr int kRowWidthMax = 32;
-__host__ __device__ constexpr int island_tile_rows(int row_width) {
+__host__ __device__ constexpr int short_row_tile_rows(int row_width) {
     return row_width > kTileMinRows ? row_width : kTileMinRows;
-}
-static_assert(2 * kWave + 4 * kIslandMaxDofs <= kTileMinRows * kTileStride, "the island search uses the row tile");
-__host__ __device__ constexpr int row_group_max(int n_equalities, int n_dofs, int max_contacts) {
-    return (6 * n_equalities + 2 * n_dofs + max_contacts + 3) / 4 * 4;
 }
 __host__ __device__ constexpr int tri4(int n) { return 8 * (n >> 2) * ((n >> 2) + 1) + 4 * (n & 3) * ((n >> 2) + 1); }
 

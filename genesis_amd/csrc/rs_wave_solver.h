@@ -156,7 +156,7 @@ __device__ __forceinline__ void wave_constraints(const DModel& m, const LState& 
                 for (int r = lane; r < 4 * ncont; r += kWave) contact_row(m, loc, 0, st, b, R, r >> 2, r & 3, nc, jt);
             }
         } else if (row_width > 0) {
-            uint32_t* chains = (uint32_t*)(tile + island_tile_rows(row_width) * kTileStride);
+            uint32_t* chains = (uint32_t*)(tile + short_row_tile_rows(row_width) * kTileStride);
             for (int64_t t = lane; t < (int64_t)4 * ncont * m.D; t += kWave) R.J[(size_t)nc * m.D + t] = 0.f;
             link_chains(m, chains, lane);
             const DenseChainJac dj{{tile + lane, chains, row_width, 0, 0, 0, 0}};

@@ -1,9 +1,8 @@
-"""The fused step of models with 25 to 128 dofs and short constraint rows: one substep from identical state against the
-per-stage step. Models with collision pairs take the dense solver with row masks (box-box contacts by MPR or by the
-separating-axis test), the others the island solver (rs_island_solver.h). The sizes and orders are those where their
-bookkeeping can go wrong: the smallest and the largest dof count, islands of one body, of chains and of the whole model,
-rows of every kind (connect, weld, joint equality, friction loss, contact, limit), dofs in both halves of the wavefront,
-and the packed triangles in LDS (one environment per workgroup) and in the state record (two and four)."""
+"""The fused step of models with 25 to 128 dofs: one substep from identical state against the per-stage step. The sizes and
+orders are those where the dense solver's bookkeeping (row masks, short rows staged by their columns, the packed Hessian)
+can go wrong: the smallest and the largest dof count, bodies apart, in chains and all in contact, rows of every kind
+(connect, weld, joint equality, friction loss, contact, limit), dofs in both halves of the wavefront, and one, two and four
+environments per workgroup (the packed Hessian of the largest models is in LDS with one, in the state record with more)."""
 
 from __future__ import annotations
 
@@ -64,9 +63,9 @@ def _quads(tmp_path, n, opts):
 
 
 MODELS = {
-    "boxes_apart_30": lambda t, o: _boxes(5, 0.5, o),  # islands of one body
-    "boxes_touching_30": lambda t, o: _boxes(5, 0.099, o),  # one island
-    "boxes_pairs_126": lambda t, o: _boxes(21, 0.0995, o),  # one island over both halves of the wavefront
+    "boxes_apart_30": lambda t, o: _boxes(5, 0.5, o),  # bodies apart
+    "boxes_touching_30": lambda t, o: _boxes(5, 0.099, o),  # one chain of contacts
+    "boxes_pairs_126": lambda t, o: _boxes(21, 0.0995, o),  # one chain over both halves of the wavefront
     "arms_26": lambda t, o: _arms(t, 13, o),  # friction, joint equality, limit and contact rows; two-dof entities
     "arms_128": lambda t, o: _arms(t, 64, o),  # every position of a lane used
     "loops_30": lambda t, o: _loops(t, 3, o),  # connect and weld rows
@@ -74,7 +73,7 @@ MODELS = {
 }
 
 
-# "alone": no collisions, the island solver (boxes then have no rows); the others: the dense solver
+# "alone": no collisions (boxes then have no rows); the detections differ for pairs of boxes only
 OPTIONS = {"sat": {"box_box_detection": True}, "mpr": {"box_box_detection": False}, "alone": {"enable_collision": False}}
 
 
@@ -105,3 +104,31 @@ def test_island_step_matches_the_per_stage_step(tmp_path, name, opts, epb):
     torch.cuda.synchronize()
     assert int(a["n_con"].max()) > 0 or (name, opts) == ("quadrupeds_36", "alone")  # no joint past its limit
     check_fused_matches_plain(a, b, model)
+
+
+def test_nan_pose_stays_in_its_environment(tmp_path):
+    """A NaN pose makes a weld's rows NaN in every column, also in those of bodies it does not join. Its environment
+    reports the error; its neighbours come out bit for bit as without it."""
+    from genesis_amd import runtime as rt
+
+    rt.load_library()
+    model = MODELS["loops_30"](tmp_path, OPTIONS["alone"])
+    dm = rt.DeviceModel(model)
+    slabs = []
+    for bad in (False, True):
+        s = rt.StateSlab(dm, 9)
+        gen = torch.Generator().manual_seed(3)
+        s["vel"].copy_(0.3 * torch.randn(model.n_dofs, 9, generator=gen))
+        s.forward_kinematics()
+        if bad:
+            s["links_quat"][:, 4] = float("nan")
+        print(f"[islands] loops_30 NaN pose in env 4: {bad}", flush=True)
+        s.step(1, rt.RS_MODE_FUSED)
+        torch.cuda.synchronize()
+        slabs.append(s)
+    good, bad = slabs
+    rest = [b for b in range(9) if b != 4]
+    assert int(bad["n_con"].max()) > 0
+    for name in ("qpos", "vel", "acc", "links_pos", "efc_force", "errbits"):
+        assert torch.equal(good[name][:, rest], bad[name][:, rest]), name
+    assert int(bad["errbits"][0, 4]) & rt.ERR_INVALID_FORCE_NAN
