@@ -9,6 +9,12 @@
 #include "../../include/rigidstep_arrays.h"
 #include "rs_fields.h"
 
+// How a unit declares the large functions of the step of models above 24 dofs (dense solver, kinematics): out of line or
+// inlined, whichever its kernels run faster with (rs_fused_gen.hip, rs_fused_gen_lds.hip).
+#ifndef RS_LARGE_FN
+#define RS_LARGE_FN inline
+#endif
+
 namespace rs {
 
 // ------------------------------------------------------------------------------------------------- model view

@@ -7,7 +7,7 @@ namespace rs {
 
 // forward_kinematics.py:580-736 func_forward_kinematics_entity, links l0 .. l1 - 1
 template <class S>
-__device__ inline void dev_forward_kinematics(const DModel& m, const S& st, int b, int l0, int l1) {
+__device__ RS_LARGE_FN void dev_forward_kinematics(const DModel& m, const S& st, int b, int l0, int l1) {
     for (int l = l0; l < l1; l++) {
         f3 pos = mvec3(m.link_pos, l);
         f4q quat = mquat(m.link_quat, l);

@@ -413,9 +413,10 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
     if (!m.disable_constraint) {
         const bool tiled = kPath == 1 || kPath == 4 || kPath == 6 || (kPath == 2 && fa.tiled != 0);
         wave_constraints(m, loc, st, b, R, lane, tile, tiled, fa.row_width);
-        const SquareH square{FP(loc, nt_H), m.D};
+        const SquareH<kLds> square{FP(loc, nt_H), m.D};
         if constexpr (kPath == 1) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile, square);
         else if constexpr (kPath == 4) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile, square);
+        else if constexpr (kPath == 0 && kLds) wave_solve<0>(m, loc, st, b, R, lane, tile, square);
         else if constexpr (kPath == 0) {
             if (fa.h_off >= 0) wave_solve<0>(m, loc, st, b, R, lane, tile, PackedH{slice + fa.h_off});
             else wave_solve<0>(m, loc, st, b, R, lane, tile, square);

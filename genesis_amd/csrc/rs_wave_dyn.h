@@ -584,7 +584,7 @@ __device__ inline void wave_forward_kinematics(const DModel& m, const LState& lo
 
 // forward kinematics, then COM, geoms and velocities split across lanes
 template <bool kMany>
-__device__ inline void wave_kinematics(const DModel& m, const LState& loc, int lane) {
+__device__ RS_LARGE_FN void wave_kinematics(const DModel& m, const LState& loc, int lane) {
     if (kMany && m.E > kManyEntities) {
         for (int e = lane; e < m.E; e += kWave) {
             const int l0 = m.entity_link_start[e], l1 = m.entity_link_end[e];

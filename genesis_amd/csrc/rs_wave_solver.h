@@ -294,7 +294,7 @@ __device__ inline void gemv_rows_mfma(const WorkRows& R, int nc, int D, const fl
 
 // solver.py:2620-2694 (same arithmetic as dev_update_constraint; for the matrix-core models J^T force on the matrix
 // cores and the cost's row sums reduced across the wavefront)
-__device__ inline float wave_update_constraint(const DModel& m, const LState& loc, const WorkRows& R, int lane,
+__device__ RS_LARGE_FN float wave_update_constraint(const DModel& m, const LState& loc, const WorkRows& R, int lane,
                                                float cost_in) {
     const int D = m.D;
     const int nc = LF(n_con, 0), ne = LF(n_con_eq, 0), nef = ne + LF(n_con_fl, 0);
@@ -402,12 +402,15 @@ __device__ inline void cholesky_in_place(int D, float* H, float eps, int lane) {
 // private region, or of a packed lower triangle in LDS (rows padded to 4 words). The factorisation, its rank-1 updates
 // and the triangular solves are chains of dependent accesses, and out of LDS each link of a chain is several times
 // shorter. Five stacks of four boxes x101: 5.65 M -> 4.95 M cycles a step (Hessian and factor 812 k -> 423 k).
+template <bool kLds>
 struct SquareH {
+    static constexpr bool kInLds = kLds;  // the private region is in LDS
     float* p;
     int D;
     __device__ __forceinline__ float& at(int i, int j) const { return p[(size_t)i * D + j]; }
 };
 struct PackedH {
+    static constexpr bool kInLds = false;
     float* p;
     __device__ __forceinline__ float& at(int i, int j) const { return p[tri4(i) + j]; }
 };
@@ -629,7 +632,9 @@ __device__ __forceinline__ void wave_hessian_cholesky(const DModel& m, const LSt
 // (uniformly) when an update degenerates. Models of up to 128 dofs: the row's vector stays in registers (lane: entries
 // lane and lane + 64), a ballot finds the next column it touches (a row touches few; every other column would be a round
 // trip to memory only to find a zero), and that column is loaded while the one before is worked on. Five stacks of four
-// boxes x101: 5.2 M -> 2.5 M cycles a step.
+// boxes x101: 5.2 M -> 2.5 M cycles a step. With the private region in LDS (at most about 50 dofs) the vector and the
+// factor are near, and the search for columns and the loads ahead, half of them of columns that fill in meanwhile, cost
+// more than they save: two quadrupeds x64, 1.41 M cycles a step column by column, 2.22 M with them.
 template <class HM>
 __device__ __forceinline__ bool wave_cholesky_incremental(const DModel& m, const LState& loc, const WorkRows& R,
                                                           const HM& H, int lane) {
@@ -643,7 +648,7 @@ __device__ __forceinline__ bool wave_cholesky_incremental(const DModel& m, const
             flips &= flips - 1;
             const float sign = R.active(c) ? 1.f : -1.f;
             const float sq = sqrtf(R.efc_D(c));
-            if (D <= 2 * kWave) {
+            if (!HM::kInLds && D <= 2 * kWave) {
                 float v[2], col[2] = {0.f, 0.f}, dk = 0.f;
 #pragma unroll
                 for (int h = 0; h < 2; h++) v[h] = lane + h * kWave < D ? R.jac(c, lane + h * kWave) * sq : 0.f;
@@ -1466,7 +1471,7 @@ struct TileLs {
 };
 
 template <int KD>
-__device__ inline float wave_linesearch(const DModel& m, const LState& loc, const WorkRows& R, int lane, float* tile) {
+__device__ RS_LARGE_FN float wave_linesearch(const DModel& m, const LState& loc, const WorkRows& R, int lane, float* tile) {
     const int D = m.D;
     float sn = 0.f;
     if (KD == 0 && mfma_model(D)) {
@@ -1504,7 +1509,7 @@ __device__ inline void export_row_forces(const DModel& m, const LState& loc, con
 // :3199-3237
 // H: the factor of the models with 25 to 128 dofs (KD = 0); every other model keeps its own in nt_H.
 template <int KD, class HM>
-__device__ inline void wave_solve(const DModel& m, const LState& loc, const DState& st, int b, const WorkRows& R,
+__device__ RS_LARGE_FN void wave_solve(const DModel& m, const LState& loc, const DState& st, int b, const WorkRows& R,
                                   int lane, float* tile, const HM& H) {
     const int D = m.D;
     const int nc = LF(n_con, 0);

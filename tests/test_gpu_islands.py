@@ -69,6 +69,7 @@ MODELS = {
     "arms_26": lambda t, o: _arms(t, 13, o),  # friction, joint equality, limit and contact rows; two-dof entities
     "arms_128": lambda t, o: _arms(t, 64, o),  # every position of a lane used
     "loops_30": lambda t, o: _loops(t, 3, o),  # connect and weld rows
+    "boxes_touching_48": lambda t, o: _boxes(8, 0.099, o),  # the most dofs whose private region fits in LDS, about
     "quadrupeds_36": lambda t, o: _quads(t, 2, o),  # overlapping robots: long rows, 18-dof entities
 }
 
@@ -77,16 +78,14 @@ MODELS = {
 OPTIONS = {"sat": {"box_box_detection": True}, "mpr": {"box_box_detection": False}, "alone": {"enable_collision": False}}
 
 
-@pytest.mark.parametrize("epb", [1, 2, 4])
-@pytest.mark.parametrize("name, opts", [(n, o) for n in MODELS for o in OPTIONS if o != "alone" or "boxes" not in n])
-def test_island_step_matches_the_per_stage_step(tmp_path, name, opts, epb):
+def _one_step_equals_the_per_stage_step(model, name, opts, config):
     from genesis_amd import runtime as rt
 
     rt.load_library()
-    model = MODELS[name](tmp_path, OPTIONS[opts])
     assert 24 < model.n_dofs <= 128
     dm = rt.DeviceModel(model)
-    dm.set_fused_config(epb, False, False, 0)
+    if config is not None:
+        dm.set_fused_config(*config)
     B = 17
     a = rt.StateSlab(dm, B)
     gen = torch.Generator().manual_seed(5)
@@ -104,6 +103,23 @@ def test_island_step_matches_the_per_stage_step(tmp_path, name, opts, epb):
     torch.cuda.synchronize()
     assert int(a["n_con"].max()) > 0 or (name, opts) == ("quadrupeds_36", "alone")  # no joint past its limit
     check_fused_matches_plain(a, b, model)
+    return dm.fused_config
+
+
+@pytest.mark.parametrize("epb", [1, 2, 4])
+@pytest.mark.parametrize("name, opts", [(n, o) for n in MODELS for o in OPTIONS if o != "alone" or "boxes" not in n])
+def test_island_step_matches_the_per_stage_step(tmp_path, name, opts, epb):
+    _one_step_equals_the_per_stage_step(MODELS[name](tmp_path, OPTIONS[opts]), name, opts, (epb, False, False, 0))
+
+
+@pytest.mark.parametrize("name, opts, in_lds", [
+    ("arms_26", "mpr", True), ("loops_30", "alone", True), ("boxes_touching_30", "sat", True),
+    ("quadrupeds_36", "mpr", True), ("boxes_touching_48", "sat", True), ("boxes_touching_48", "mpr", True),
+    ("boxes_pairs_126", "sat", False), ("arms_128", "alone", False)])
+def test_default_launch_shape_matches_the_per_stage_step(tmp_path, name, opts, in_lds):
+    """As a model is created: one environment per workgroup, the private region in LDS where it fits."""
+    c = _one_step_equals_the_per_stage_step(MODELS[name](tmp_path, OPTIONS[opts]), name, opts, None)
+    assert c["envs_per_block"] == 1 and c["use_lds"] == in_lds
 
 
 def test_nan_pose_stays_in_its_environment(tmp_path):
