@@ -27,7 +27,7 @@ FLAGS = [
 
 # translation units: the C ABI with the per-stage kernels, and one unit per fused-kernel class (compiled in parallel)
 SOURCES = ["rs_lib.hip", "rs_fused_t16.hip", "rs_fused_t24.hip", "rs_fused_gen.hip",
-           "rs_fused_gen_lds.hip", "rs_fused_multi.hip"]
+           "rs_fused_gen_lds.hip", "rs_fused_multi.hip", "rs_fused_multi_any.hip"]
 OBJ_DIR = os.path.join(HERE, "_build")
 
 

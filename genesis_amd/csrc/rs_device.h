@@ -9,8 +9,8 @@
 #include "../../include/rigidstep_arrays.h"
 #include "rs_fields.h"
 
-// How a unit declares the large functions of the step of models above 24 dofs (dense solver, kinematics): out of line or
-// inlined, whichever its kernels run faster with (rs_fused_gen.hip, rs_fused_gen_lds.hip).
+// How a unit declares the functions of the step of models above 24 dofs that are called more than once or stand apart from
+// the solver (row update, kinematics): out of line or inlined, whichever its kernels run faster with.
 #ifndef RS_LARGE_FN
 #define RS_LARGE_FN inline
 #endif
@@ -21,6 +21,7 @@ namespace rs {
 // Model arrays are read-only while kernels run, so they live in the constant address space: reads at addresses that
 // are the same on every lane become scalar loads.
 #define RS_CONST __attribute__((address_space(4)))
+#define RS_LDS __attribute__((address_space(3)))
 typedef const float RS_CONST* cfptr;
 typedef const int32_t RS_CONST* ciptr;
 

@@ -364,8 +364,8 @@ __device__ inline void wave_integrate(const DModel& m, const LState& loc, int la
 
 // One environment's substep on the calling wavefront (w = wavefront index in the workgroup).
 // kPath: 1 = models in the first row-tile class (at most kTileMaxDofs dofs), 4 = the second (up to kTileWideDofs),
-// 0 = larger models; decided per call (the shared launch of
-// several models): 2 = any, 6 = models of up to kTileWideDofs. Returns the narrowphase's GJK/EPA work (see
+// 0 = larger models with the Hessian in the private region, 3 = with the packed Hessian in LDS; 6 = either row-tile
+// class, decided per call (shared launches of several models). Returns the narrowphase's GJK/EPA work (see
 // wave_narrowphase).
 template <bool kLds, int kPath>
 __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, const FusedArgs& fa,
@@ -390,7 +390,7 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
     if constexpr (kPath == 1 || kPath == 4)
         if (FP(loc, n_con)[0] >= kSchedHeavyRows) __builtin_amdgcn_s_setprio(3);
     // kernel_step_1: CRBA, L^T D L, actuation + passive + bias forces, acc_smooth
-    constexpr bool kMany = kPath != 1 && kPath != 4 && kPath != 6;
+    constexpr bool kMany = kPath == 0 || kPath == 3;
     wave_mass_matrix<kMany>(m, loc, lane);
     wave_factor_mass(m, loc, lane);
     wave_torque_passive(m, loc, lane);
@@ -411,21 +411,14 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
     }
     // ConstraintSolver.resolve
     if (!m.disable_constraint) {
-        const bool tiled = kPath == 1 || kPath == 4 || kPath == 6 || (kPath == 2 && fa.tiled != 0);
-        wave_constraints(m, loc, st, b, R, lane, tile, tiled, fa.row_width);
+        wave_constraints(m, loc, st, b, R, lane, tile, !kMany, fa.row_width);
         const SquareH<kLds> square{FP(loc, nt_H), m.D};
         if constexpr (kPath == 1) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile, square);
         else if constexpr (kPath == 4) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile, square);
-        else if constexpr (kPath == 0 && kLds) wave_solve<0>(m, loc, st, b, R, lane, tile, square);
-        else if constexpr (kPath == 0) {
-            if (fa.h_off >= 0) wave_solve<0>(m, loc, st, b, R, lane, tile, PackedH{slice + fa.h_off});
-            else wave_solve<0>(m, loc, st, b, R, lane, tile, square);
-        } else if (fa.tiled == kTileMaxDofs) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile, square);
-        else if (kPath == 6 || fa.tiled == kTileWideDofs) wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile, square);
-        else if constexpr (kPath == 2) {
-            if (fa.h_off >= 0) wave_solve<0>(m, loc, st, b, R, lane, tile, PackedH{slice + fa.h_off});
-            else wave_solve<0>(m, loc, st, b, R, lane, tile, square);
-        }
+        else if constexpr (kPath == 0) wave_solve<0>(m, loc, st, b, R, lane, tile, square);
+        else if constexpr (kPath == 3) wave_solve<0>(m, loc, st, b, R, lane, tile, PackedH{slice + fa.h_off});
+        else if (fa.tiled == kTileMaxDofs) wave_solve<kTileMaxDofs>(m, loc, st, b, R, lane, tile, square);
+        else wave_solve<kTileWideDofs>(m, loc, st, b, R, lane, tile, square);
     }
     // kernel_step_2: cacc, semi-implicit Euler, forward kinematics and velocities
     wave_update_acc<kMany>(m, loc, lane, true);
@@ -512,7 +505,7 @@ k_fused_wave(DModel m, DState st, FusedArgs fa) {
     fused_launch<kLds, kPath>(m, st, fa, (const RS_CONST int*)fa.loc_off);
 }
 
-// Models above 24 dofs (kPath 0): at most kGenericMaxThreads lanes (4 environments) per workgroup, so that a
+// Models above 24 dofs (kPath 0 and 3): at most kGenericMaxThreads lanes (4 environments) per workgroup, so that a
 // wavefront may hold all 512 registers of its SIMD.
 template <bool kLds, int kPath>
 __global__ void __launch_bounds__(kGenericMaxThreads) k_fused_large(FusedKernArgs) {
@@ -528,14 +521,25 @@ struct FusedSegment {
     int first_block, n_blocks;
 };
 
+// One environment of a larger model in a shared launch: a function of its own, so that its registers are allocated for it
+// alone (in one body with the row-tile solvers it spills: 1024 piles 14.2 to 15.1 ms for 4 ticks, 10.5 so; 1500 quadrupeds,
+// 500 arms and 150 piles 10.6 and 8.3 ms). The arguments of a call arrive per lane; they are the same on every lane.
+template <int kPath>
+__device__ __attribute__((noinline)) inline void shared_large_env(const FusedSegment* seg, int env, RS_LDS float* lds) {
+    const uint64_t at = (uint64_t)(uintptr_t)seg;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)at), hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
+    const RS_CONST FusedSegment* g = (const RS_CONST FusedSegment*)(uintptr_t)((uint64_t)hi << 32 | lo);
+    const FusedSegment& s = *(const FusedSegment*)g;
+    RS_LDS float* base = (RS_LDS float*)(uintptr_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
+    fused_env<false, kPath>(s.m, s.st, s.fa, g->fa.loc_off, __builtin_amdgcn_readfirstlane(env), 0, (float*)base);
+}
+
 // Several models and slabs in one launch (the serving loop's co-batched step). Every segment uses the launch's
 // environments-per-workgroup; a workgroup finds its segment by scanning the table (a few dozen entries at most).
-// kPath 6: every model has a row tile. kPath 2: some model has more than 24 dofs; its environments are the longest, so
-// the launch gives every wavefront all registers of its SIMD and room for the Hessian in LDS, and keeps the private
-// regions in memory (1000 quadrupeds, 333 arms and 100 piles: 10.9 -> 10.3 ms for 4 ticks, against two wavefronts per
-// SIMD; 8 piles with 16384 quadrupeds, which would rather have the second wavefront, 21.8 -> 22.9 ms).
-template <bool kLds, int kPath>
-__global__ void __launch_bounds__(kPath == 2 ? kWave : 512)
+// kLarge: some model has more than 24 dofs; its environments are the longest, so the launch gives every wavefront all
+// registers of its SIMD and room for the Hessian in LDS, and keeps the private regions in memory.
+template <bool kLds, bool kLarge>
+__global__ void __launch_bounds__(kLarge ? kWave : 512)
 k_fused_multi(const FusedSegment* __restrict__ segs, int n_segs) {
     extern __shared__ float lds_env[];
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -543,13 +547,18 @@ k_fused_multi(const FusedSegment* __restrict__ segs, int n_segs) {
     // The table does not change while the kernel runs: read through the constant address space, its entries (the model's
     // and the slab's pointers among them) are scalar loads.
     const FusedSegment* tab = segs;
-    if constexpr (kPath == 2) tab = (const FusedSegment*)(const RS_CONST FusedSegment*)(uintptr_t)segs;
+    if constexpr (kLarge) tab = (const FusedSegment*)(const RS_CONST FusedSegment*)(uintptr_t)segs;
     int s = 0;
     while (s + 1 < n_segs && tab[s + 1].first_block <= blk) s++;
     const FusedSegment& g = tab[s];
     const int b = (blk - g.first_block) * g.fa.epb + w;
     if (b >= g.st.B) return;
-    fused_env<kLds, kPath>(g.m, g.st, g.fa, (const RS_CONST int*)g.fa.loc_off, b, w, lds_env);
+    if (!kLarge || g.fa.tiled) {
+        fused_env<kLds, 6>(g.m, g.st, g.fa, (const RS_CONST int*)g.fa.loc_off, b, w, lds_env);
+    } else if constexpr (kLarge) {
+        if (g.fa.h_off >= 0) shared_large_env<3>(segs + s, b, (RS_LDS float*)lds_env);
+        else shared_large_env<0>(segs + s, b, (RS_LDS float*)lds_env);
+    }
 }
 
 }  // namespace rs

@@ -1,6 +1,6 @@
 // Host-side launchers of the fused substep kernels. Each kernel class is instantiated in a translation unit of its own
 // (rs_fused_t16.hip, rs_fused_t24.hip, rs_fused_gen.hip, rs_fused_gen_lds.hip,
-// rs_fused_multi.hip) so that the library builds in parallel.
+// rs_fused_multi.hip, rs_fused_multi_any.hip) so that the library builds in parallel.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -19,8 +19,9 @@ void launch_fused_generic(bool use_lds, dim3 grid, dim3 block, size_t lds_bytes,
                           const DState& st, const FusedArgs& fa);
 void launch_fused_generic_lds(dim3 grid, dim3 block, size_t lds_bytes, hipStream_t s, const DModel& m, const DState& st,
                               const FusedArgs& fa);
-// k_fused_multi: one fused substep of several (model, slab) segments
-void launch_fused_multi(bool use_lds, bool large, dim3 grid, dim3 block, size_t lds_bytes, hipStream_t s,
+// k_fused_multi: one fused substep of several (model, slab) segments, of models with a row tile or of any
+void launch_fused_multi(bool use_lds, dim3 grid, dim3 block, size_t lds_bytes, hipStream_t s,
                         const FusedSegment* segs, int n_segs);
+void launch_fused_multi_any(dim3 grid, dim3 block, size_t lds_bytes, hipStream_t s, const FusedSegment* segs, int n_segs);
 
 }  // namespace rs

@@ -956,7 +956,8 @@ int rs_batch_step(rs_batch* bt, int n, const rs_model* const* models, void* cons
     HIP_OK(hipEventRecord(bt->done[k], s));
     bt->pending[k] = true;
     const dim3 grid((unsigned)blocks), block((unsigned)(kWave * epb));
-    launch_fused_multi(use_lds, large, grid, block, (size_t)epb * slice * 4, s, bt->dev[k], n);
+    if (large) launch_fused_multi_any(grid, block, (size_t)epb * slice * 4, s, bt->dev[k], n);
+    else launch_fused_multi(use_lds, grid, block, (size_t)epb * slice * 4, s, bt->dev[k], n);
     HIP_OK(hipGetLastError());
     return RS_OK;
 }

@@ -1471,7 +1471,7 @@ struct TileLs {
 };
 
 template <int KD>
-__device__ RS_LARGE_FN float wave_linesearch(const DModel& m, const LState& loc, const WorkRows& R, int lane, float* tile) {
+__device__ __forceinline__ float wave_linesearch(const DModel& m, const LState& loc, const WorkRows& R, int lane, float* tile) {
     const int D = m.D;
     float sn = 0.f;
     if (KD == 0 && mfma_model(D)) {
@@ -1509,7 +1509,7 @@ __device__ inline void export_row_forces(const DModel& m, const LState& loc, con
 // :3199-3237
 // H: the factor of the models with 25 to 128 dofs (KD = 0); every other model keeps its own in nt_H.
 template <int KD, class HM>
-__device__ RS_LARGE_FN void wave_solve(const DModel& m, const LState& loc, const DState& st, int b, const WorkRows& R,
+__device__ __forceinline__ void wave_solve(const DModel& m, const LState& loc, const DState& st, int b, const WorkRows& R,
                                   int lane, float* tile, const HM& H) {
     const int D = m.D;
     const int nc = LF(n_con, 0);

@@ -65,3 +65,12 @@ def test_row_tile_and_lds_kernels_hold_their_functions_inlined():
         for n in called:
             if "k_sched_flip" not in n:
                 assert not any(t in n for t in ("DModel", "DState", "LState", "FusedArgs", "WorkRows")), n
+
+
+def test_no_kernel_calls_its_solver():
+    runtime.load_library()
+    units = list(_fused_units())
+    assert len(units) == 6
+    for kernels, functions in units:
+        solver = [n for n in functions if "wave_solve" in n or "wave_linesearch" in n or "cholesky" in n]
+        assert not solver, (sorted(kernels), solver)
