@@ -314,7 +314,8 @@ class StepGraph:
 
 
 class SharedLaunch:
-    """One fused substep of several slabs (of possibly different models) in a single kernel launch (rs_batch)."""
+    """One fused substep of several slabs (of possibly different models) in one kernel launch, or two side by
+    side (rs_batch)."""
 
     def __init__(self, max_segments: int = 64):
         lib = load_library()

@@ -228,7 +228,8 @@ int rs_fused_config_get(const rs_model* model, rs_fused_config* out);
 int rs_fused_config_set(rs_model* model, const rs_fused_config* config);
 
 /* Shared launches for serving: one fused substep of n independent batches - each a model, its state slab and its
- * environment count, models may differ - in a single kernel launch. Each environment's result is the same as when
+ * environment count, models may differ - in a single kernel launch, or, where models above 24 dofs meet many small
+ * environments, in two side by side (the second on a stream of the batch's own, which `stream` waits for). Each environment's result is the same as when
  * its slab is stepped alone with rs_step(RS_MODE_FUSED). The batch object owns a ring of four small pinned/device
  * segment tables (up to max_segments entries each); rs_batch_step waits only for the table copy it issued four calls
  * earlier before reusing that table. No counterpart in the reference (its scenes step one at a time). */
