@@ -75,10 +75,22 @@ __host__ __device__ constexpr bool is_local_kind(int kind) {
 // One environment's private-region fields (fused kernel): field F starts at base + off[F] and has row stride 1. The
 // offsets stay in kernel-argument (constant) memory and every access computes its address from them, so the view
 // holds two uniform values instead of a pointer per field.
+// LocOffsets: how a kernel reaches them. Kernels that take their arguments by value (RS_ARGS_BY_VALUE) use an ordinary
+// pointer, whose memory the compiler finds by itself: with the arguments in place the offsets are scalar loads; were they
+// copied to scratch memory, the offsets would be scratch loads, whereas such a copy's address cast to the constant address
+// space is one that scalar loads fault on. The other kernels have their arguments from a pointer to constant memory, and
+// say so, since functions called out of line cannot find it.
+#ifdef RS_ARGS_BY_VALUE
+typedef const int* LocOffsets;
+constexpr bool kArgsByValue = true;
+#else
+typedef const RS_CONST int* LocOffsets;
+constexpr bool kArgsByValue = false;
+#endif
 struct LState {
     static constexpr int B = 1;
     float* base;
-    const RS_CONST int* off;
+    LocOffsets off;
 };
 
 template <int F>

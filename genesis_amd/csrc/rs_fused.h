@@ -368,8 +368,8 @@ __device__ inline void wave_integrate(const DModel& m, const LState& loc, int la
 // class, decided per call (shared launches of several models). Returns the narrowphase's GJK/EPA work (see
 // wave_narrowphase).
 template <bool kLds, int kPath>
-__device__ __forceinline__ int fused_env(const DModel& m, const DState& st, const FusedArgs& fa,
-                                          const RS_CONST int* loc_off, int b, int w, float* lds_env) {
+__device__ __forceinline__ int fused_env(const DModel& m, const DState& st, const FusedArgs& fa, int b, int w,
+                                         float* lds_env) {
     const int lane = lane_id();
     float* wk = st.wk + (size_t)b * fa.work_stride;
     float* slice = lds_env + (size_t)w * fa.lds_wave;
@@ -379,7 +379,7 @@ __device__ __forceinline__ int fused_env(const DModel& m, const DState& st, cons
     const bool in_place = !kLds && st.LS > 0;
     float* base = kLds ? slice : in_place ? (float*)((uint32_t*)(void*)st.qpos + (size_t)b * st.LS) : wk + fa.off_loc;
     float* tile = slice + fa.tile_off;
-    const LState loc = make_local(base, loc_off);
+    const LState loc = make_local(base, (LocOffsets)fa.loc_off);
     const WorkRows R{wk + fa.off_jac, wk + fa.off_rowf, wk + fa.off_tmp, m.CMAX, m.D};
 
     if (!in_place) stage_local<true>(st, (uint32_t*)base, fa.n_local, b, lane);
@@ -446,10 +446,9 @@ static __global__ void k_sched_flip(DState st) {
 // The arguments of a launch for larger models, which its kernels reach through the kernel-argument segment's own pointer.
 // A parameter passed by value is copied to every lane's scratch memory as soon as the compiler forms one pointer to two of
 // its members (two branches that read different members are enough) or a function that takes it by reference is not
-// inlined. Then every model array's address comes from a vector load of scratch memory instead of a scalar load, and
-// LState's offsets, cast to the constant address space from such a copy, are an address that scalar loads fault on. The
-// kernels of the smaller models take theirs by value (5% faster: the compiler may load those ahead of a branch) and must
-// keep all their functions inlined.
+// inlined. Then every model array's address comes from a vector load of scratch memory instead of a scalar load. The
+// kernels of the smaller models take theirs by value (through the segment's pointer they are 3 to 5% slower: the compiler
+// may load those ahead of a branch).
 struct FusedKernArgs {
     DModel m;
     DState st;
@@ -461,8 +460,7 @@ __device__ __forceinline__ const RS_CONST FusedKernArgs* kern_args() {
 
 // the wavefront's environment of a launch: blockIdx order, or the schedule's
 template <bool kLds, int kPath>
-__device__ __forceinline__ void fused_launch(const DModel& m, const DState& st, const FusedArgs& fa,
-                                             const RS_CONST int* loc_off) {
+__device__ __forceinline__ void fused_launch(const DModel& m, const DState& st, const FusedArgs& fa) {
     extern __shared__ float lds_env[];
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     int b = xcd_block((int)blockIdx.x, (int)gridDim.x) * fa.epb + w;
@@ -488,7 +486,7 @@ __device__ __forceinline__ void fused_launch(const DModel& m, const DState& st, 
         }
     }
     if (b >= st.B) return;  // whole wavefronts only
-    const int gjk_work = fused_env<kLds, kPath>(m, st, fa, loc_off, b, w, lds_env);
+    const int gjk_work = fused_env<kLds, kPath>(m, st, fa, b, w, lds_env);
     if (fa.sched && lane_id() == 0) {
         const int cls = sched_class(FV(st, n_con, b)[0], gjk_work);
         const int q = par ^ 1;
@@ -502,7 +500,8 @@ __device__ __forceinline__ void fused_launch(const DModel& m, const DState& st, 
 template <bool kLds, int kOcc, int kPath>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kOcc > 0 ? kOcc : 1, 8)))
 k_fused_wave(DModel m, DState st, FusedArgs fa) {
-    fused_launch<kLds, kPath>(m, st, fa, (const RS_CONST int*)fa.loc_off);
+    static_assert(kArgsByValue || kPath < 0, "a cast of the arguments' address to constant memory is not safe here");
+    fused_launch<kLds, kPath>(m, st, fa);
 }
 
 // Models above 24 dofs (kPath 0 and 3): at most kGenericMaxThreads lanes (4 environments) per workgroup, so that a
@@ -510,7 +509,8 @@ k_fused_wave(DModel m, DState st, FusedArgs fa) {
 template <bool kLds, int kPath>
 __global__ void __launch_bounds__(kGenericMaxThreads) k_fused_large(FusedKernArgs) {
     const FusedKernArgs& a = *(const FusedKernArgs*)kern_args();
-    fused_launch<kLds, kPath>(a.m, a.st, a.fa, kern_args()->fa.loc_off);
+    static_assert(!kArgsByValue || kPath < 0, "the arguments are in constant memory");
+    fused_launch<kLds, kPath>(a.m, a.st, a.fa);
 }
 
 // One batch of a shared launch: a model, its state slab, and the first workgroup that serves it.
@@ -531,7 +531,7 @@ __device__ __attribute__((noinline)) inline void shared_large_env(const FusedSeg
     const RS_CONST FusedSegment* g = (const RS_CONST FusedSegment*)(uintptr_t)((uint64_t)hi << 32 | lo);
     const FusedSegment& s = *(const FusedSegment*)g;
     RS_LDS float* base = (RS_LDS float*)(uintptr_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-    fused_env<false, kPath>(s.m, s.st, s.fa, g->fa.loc_off, __builtin_amdgcn_readfirstlane(env), 0, (float*)base);
+    fused_env<false, kPath>(s.m, s.st, s.fa, __builtin_amdgcn_readfirstlane(env), 0, (float*)base);
 }
 
 // Several models and slabs in one launch (the serving loop's co-batched step). Every segment uses the launch's
@@ -554,7 +554,7 @@ k_fused_multi(const FusedSegment* __restrict__ segs, int n_segs) {
     const int b = (blk - g.first_block) * g.fa.epb + w;
     if (b >= g.st.B) return;
     if (!kLarge || g.fa.tiled) {
-        fused_env<kLds, 6>(g.m, g.st, g.fa, (const RS_CONST int*)g.fa.loc_off, b, w, lds_env);
+        fused_env<kLds, 6>(g.m, g.st, g.fa, b, w, lds_env);
     } else if constexpr (kLarge) {
         if (g.fa.h_off >= 0) shared_large_env<3>(segs + s, b, (RS_LDS float*)lds_env);
         else shared_large_env<0>(segs + s, b, (RS_LDS float*)lds_env);

@@ -1,5 +1,6 @@
 // Fused substep kernels of models with at most 16 dofs (row tile of 16): private region in LDS or in the work field,
 // occupancy 0 (compiler's register budget), 3 or 4 wavefronts per SIMD.
+#define RS_ARGS_BY_VALUE
 #include "rs_launch.h"
 
 namespace rs {

@@ -1,4 +1,5 @@
 // Fused substep kernels of models with 17 to 24 dofs (row tile of 24): occupancy 0 or 3.
+#define RS_ARGS_BY_VALUE
 #include "rs_launch.h"
 
 namespace rs {

@@ -196,9 +196,8 @@ __device__ __forceinline__ void tile_seq_sums(float& acc, const float (&v)[NQ], 
 }
 
 // ---------------------------------------------------------------------------------------- private region
-// the local view of the environment whose private region starts at base; off: the field offsets in constant memory (the
-// kernel-argument segment or a launch's table)
-__device__ __forceinline__ LState make_local(float* base, const RS_CONST int* off) {
+// the local view of the environment whose private region starts at base; off: the field offsets (FusedArgs::loc_off)
+__device__ __forceinline__ LState make_local(float* base, LocOffsets off) {
     return LState{base, off};
 }
 
