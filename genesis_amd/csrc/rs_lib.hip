@@ -178,6 +178,12 @@ static void set_lds_slice(const rs_model_header& h, FusedArgs* fa, bool use_lds,
 static int lds_slice_floats(const rs_model_header& h, const FusedArgs& fa, bool use_lds) {
     return (use_lds ? fa.loc_floats : 0) + tile_floats(h, fa) + fa.gjk_words;
 }
+// Short rows need four words of LDS per link and, above kTileMinRows columns, a taller tile. Where that is what makes a
+// launch not fit (a few dofs among some hundred fixed links, say), it builds its contact rows dense: the same rows.
+static FusedArgs rows_that_fit(const rs_model_header& h, FusedArgs fa, int epb, bool use_lds, int max_lds) {
+    if ((int64_t)epb * lds_slice_floats(h, fa, use_lds) * 4 > max_lds) fa.row_width = 0;
+    return fa;
+}
 // the packed lower triangle of the Hessian of models above 24 dofs follows in the slice when the workgroup's slices still
 // fit with it (it is in nt_H otherwise): every step of a factorisation or a triangular solve waits for a round trip to it
 static int slice_with_hessian(const rs_model* m, const FusedArgs& fa, bool use_lds, int* h_off, int max_lds) {
@@ -473,6 +479,7 @@ static int fused_substep(const rs_model* m, const DState& st, hipStream_t s) {
     fa.sched = m->schedule && st.B >= sched_rows();
     if (fa.sched) hipLaunchKernelGGL(k_sched_flip, dim3(1), dim3(1), 0, s, st);
     const dim3 grid((unsigned)((st.B + epb - 1) / epb)), block((unsigned)(kWave * epb));
+    fa = rows_that_fit(m->h, fa, epb, m->use_lds, m->max_lds);
     int h_off = -1;
     set_lds_slice(m->h, &fa, m->use_lds, slice_with_hessian(m, fa, m->use_lds, &h_off, m->max_lds));
     fa.h_off = h_off;
@@ -492,7 +499,8 @@ static int check_fused_config(const rs_model* m, const FusedArgs& fa, int epb, i
     if (epb < 1 || epb > 8) return fail(RS_E_INVALID, "fused config: envs_per_block must be in 1..8");
     if (!m->fa.tiled && epb * kWave > kGenericMaxThreads)
         return fail(RS_E_UNSUPPORTED, "fused config: models above 24 dofs run at most 4 environments per workgroup");
-    if ((int64_t)epb * lds_slice_floats(m->h, fa, use_lds) * 4 > m->max_lds)
+    const FusedArgs fit = rows_that_fit(m->h, fa, epb, use_lds, m->max_lds);
+    if ((int64_t)epb * lds_slice_floats(m->h, fit, use_lds) * 4 > m->max_lds)
         return fail(RS_E_UNSUPPORTED, use_lds ? "fused config: private regions do not fit in LDS at this envs_per_block"
                                               : "fused config: row tiles do not fit in LDS at this envs_per_block");
     return RS_OK;
@@ -667,7 +675,8 @@ int rs_fused_config_get(const rs_model* m, rs_fused_config* out) {
     out->envs_per_block = m->fa.epb;
     out->use_lds = m->use_lds;
     int h_off;
-    out->lds_bytes_per_env = slice_with_hessian(m, m->fa, m->use_lds, &h_off, m->max_lds) * 4;
+    const FusedArgs fit = rows_that_fit(m->h, m->fa, m->fa.epb, m->use_lds, m->max_lds);
+    out->lds_bytes_per_env = slice_with_hessian(m, fit, m->use_lds, &h_off, m->max_lds) * 4;
     out->schedule = m->schedule;
     out->occupancy = m->occupancy;
     out->gjk_lds = m->fa.gjk_words > 0;
@@ -976,7 +985,7 @@ int rs_batch_step(rs_batch* bt, int n, const rs_model* const* models, void* cons
             FusedSegment& g = tab[at++];
             g.m = models[i]->dm;
             g.st = make_state(models[i], states[i], n_envs[i]);
-            g.fa = models[i]->fa;
+            g.fa = l.use_lds ? models[i]->fa : rows_that_fit(models[i]->h, models[i]->fa, l.epb, false, max_lds);
             g.fa.epb = l.epb;
             int h_off = -1;
             const int own = l.use_lds ? slice_lds : slice_with_hessian(models[i], g.fa, false, &h_off, max_lds);

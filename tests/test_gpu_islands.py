@@ -191,3 +191,29 @@ def test_shared_launch_of_both_classes_equals_the_launches_alone(tmp_path, n_sma
         for name in ("qpos", "acc", "n_con", "errbits"):
             assert torch.equal(a[name], b[name]), (a.dmodel.model.n_dofs, name)
     assert all(int(b["n_con"].max()) > 0 for b in mixed[1:])
+
+
+def _frames(tmp_path, n):
+    """n bodies without joints, one entity."""
+    p = os.path.join(str(tmp_path), f"frames{n}.xml")
+    with open(p, "w") as f:
+        f.write('<mujoco model="frames"><worldbody><body name="r" pos="5 0 0">')
+        for i in range(n):
+            f.write(f'<body name="f{i}" pos="0 {0.01 * i} 0"><inertial pos="0 0 0" mass="0.1" '
+                    'diaginertia="0.001 0.001 0.001"/></body>')
+        f.write("</body></worldbody></mujoco>")
+    return load_mjcf(p, "frames")
+
+
+@pytest.mark.parametrize("n_links", [64, 900])
+def test_rows_are_built_dense_where_their_staging_does_not_fit(tmp_path, n_links):
+    """Four environments per workgroup, contact rows staged with four LDS words per link: with 900 links that does not fit,
+    and the launch is accepted all the same."""
+    ents = [plane_entity(friction=0.5), _frames(tmp_path, n_links)]
+    for i in range(5):
+        ents.append(box_entity(np.full(3, 0.1), np.array([0.099 * i, 0.01 * (i % 3), 0.049]), np.array([1.0, 0, 0, 0]),
+                               rho=500.0, friction=0.5, name=f"b{i}"))
+    model = compile_model(ents, SolverOptions(dt=0.01, box_box_detection=True))
+    assert model.n_links > n_links and model.n_dofs == 30
+    c = _one_step_equals_the_per_stage_step(model, "boxes", "sat", (4, False, False, 0))
+    assert c["envs_per_block"] == 4 and not c["use_lds"] and 4 * c["lds_bytes_per_env"] <= 65536
