@@ -664,6 +664,10 @@ int rs_model_update(rs_model* m, const rs_model_header* h, const void* blob, siz
     if (blob_bytes != m->blob_bytes || std::memcmp(h, &m->h, sizeof(rs_model_header)) != 0)
         return fail(RS_E_INVALID, "rs_model_update: the header or blob size differs from the model's (only array "
                                   "values may change)");
+    // launches (and captured graphs) stage contact rows of up to row_width dofs
+    const int width = short_row_width(*h, (const char*)blob);
+    if (m->fa.row_width > 0 && (width == 0 || width > m->fa.row_width))
+        return fail(RS_E_INVALID, "rs_model_update: the links' tree has longer chains of dofs than the model's");
     hipStream_t s = (hipStream_t)stream;
     HIP_OK(hipMemcpyAsync(m->blob, blob, blob_bytes, hipMemcpyHostToDevice, s));
     HIP_OK(hipStreamSynchronize(s));

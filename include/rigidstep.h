@@ -134,7 +134,8 @@ void rs_model_destroy(rs_model* model);
 
 /* Overwrite the model's array values with a blob of the same header (counts, options and offsets unchanged), in
  * stream order, then synchronise the stream; the device address, the launch configuration and captured graphs stay
- * valid and see the new values. Used by the dof parameter setters (set_dofs_kp / kv / force_range / damping /
+ * valid and see the new values. Refused: a tree of links with longer chains of dofs than the created model's, which its
+ * launches have no room for. Used by the dof parameter setters (set_dofs_kp / kv / force_range / damping /
  * stiffness, engine/entities/rigid_entity/rigid_entity.py:3372-3500, which write dofs_info in place). */
 int rs_model_update(rs_model* model, const rs_model_header* header, const void* blob, size_t blob_bytes, void* stream);
 

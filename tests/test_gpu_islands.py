@@ -217,3 +217,21 @@ def test_rows_are_built_dense_where_their_staging_does_not_fit(tmp_path, n_links
     assert model.n_links > n_links and model.n_dofs == 30
     c = _one_step_equals_the_per_stage_step(model, "boxes", "sat", (4, False, False, 0))
     assert c["envs_per_block"] == 4 and not c["use_lds"] and 4 * c["lds_bytes_per_env"] <= 65536
+
+
+def test_update_refuses_a_tree_with_longer_chains():
+    """Launches stage rows of as many dofs as two of the created model's chains have; a box hung under another would double
+    them. Other values are updated as before."""
+    from genesis_amd import runtime as rt
+
+    rt.load_library()
+    model = _boxes(5, 0.5, OPTIONS["sat"])
+    dm = rt.DeviceModel(model)
+    parent = model.arrays["link_parent"]
+    keep = parent.copy()
+    parent[3] = 2
+    with pytest.raises(rt.RigidStepError, match="longer chains"):
+        dm.update()
+    parent[:] = keep
+    model.arrays["geom_friction"][:] = 0.7
+    dm.update()
