@@ -29,7 +29,7 @@ struct FusedArgs {
     int gjk_words;     // LDS floats per wavefront for the GJK/EPA polytope (0: the polytope stays in the work field)
     int gjk_off;       // offset of that polytope in the wavefront's LDS slice (-1: none)
     int tile_off;      // offset of the row tile (kTileStride x tile_rows(D) floats) in the wavefront's LDS slice
-    int row_width;     // most dofs a constraint row touches, a multiple of 4 (models with 25 to 128 dofs; 0: over 32)
+    int row_width;     // most dofs a constraint row touches, a multiple of 4 (25 to 128 dofs; 0: over 32, or no room)
     int h_off;         // offset of the packed Hessian of models above 24 dofs in the wavefront's LDS slice (-1: in nt_H)
     int sched;         // 1: map wavefronts to environments through the cost-ordered queues
     int loc_off[kMaxStateFields];  // private-region offset of each state field (local kinds only)

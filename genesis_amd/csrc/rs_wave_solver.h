@@ -210,7 +210,9 @@ __device__ __forceinline__ float wave_dsum(int D, int lane, F f) {
 }
 
 // union of the tile masks of rows c0 .. c0 + n - 1 (uniform). A product with a tile in which every row is zero adds
-// exactly nothing to its accumulators, so it is left out, loads and all: of a pile's 8 tiles a contact touches 1 to 4.
+// exactly nothing to its accumulators, so it is left out, loads and all: of a pile's 8 tiles a contact touches 1 to 4. (A
+// weight that is not finite would add NaN to it; the triangular solves, which are dense, spread it to every dof all the
+// same.)
 __device__ __forceinline__ int tiles_of_rows(const WorkRows& R, int nc, int c0, int n, int lane) {
     const int mine = lane < n && c0 + lane < nc ? R.tiles(c0 + lane) : 0;
     int on = 0;

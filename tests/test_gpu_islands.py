@@ -151,6 +151,35 @@ def test_nan_pose_stays_in_its_environment(tmp_path):
     assert int(bad["errbits"][0, 4]) & rt.ERR_INVALID_FORCE_NAN
 
 
+@pytest.mark.parametrize("name, in_lds", [("boxes_apart_30", True), ("boxes_apart_30", False), ("boxes_pairs_126", False)])
+def test_nan_velocity_spreads_as_in_the_per_stage_step(tmp_path, name, in_lds):
+    """Products leave out the tiles in which every row is zero, where a row force that is not a number would have added one:
+    the environment's accelerations, forces and error bits are those of the per-stage step all the same."""
+    from genesis_amd import runtime as rt
+
+    rt.load_library()
+    model = MODELS[name](tmp_path, OPTIONS["sat"])
+    dm = rt.DeviceModel(model)
+    dm.set_fused_config(1, in_lds, False, 0)
+    a = rt.StateSlab(dm, 5)
+    gen = torch.Generator().manual_seed(5)
+    a["vel"].copy_(0.3 * torch.randn(model.n_dofs, 5, generator=gen))
+    a.forward_kinematics()
+    a.step(3, rt.RS_MODE_PLAIN)
+    torch.cuda.synchronize()
+    a["vel"][model.n_dofs - 2, 2] = float("nan")
+    b = rt.StateSlab(dm, 5)
+    b.buffer.copy_(a.buffer)
+    print(f"[islands] {name} NaN velocity of the last body in env 2, config={dm.fused_config}", flush=True)
+    a.step(1, rt.RS_MODE_PLAIN)
+    b.step(1, rt.RS_MODE_FUSED)
+    torch.cuda.synchronize()
+    assert torch.equal(a["errbits"], b["errbits"]) and int(b["errbits"][0, 2]) & rt.ERR_INVALID_FORCE_NAN
+    for field in ("acc", "qacc_ws", "qf_constraint", "vel", "qpos"):
+        assert torch.equal(a[field].isnan(), b[field].isnan()), field
+    assert torch.equal(a["qpos"][:, 2], b["qpos"][:, 2])  # the NaN guard kept the old pose
+
+
 @pytest.mark.parametrize("n_small", [33, 2100])
 def test_shared_launch_of_both_classes_equals_the_launches_alone(tmp_path, n_small):
     """Row-tile models and larger ones (region in LDS when alone, collision-free, the most dofs of the matrix-core path, and
