@@ -27,6 +27,7 @@ sys.path.insert(0, REPO)
 
 from genesis_amd import runtime as rt  # noqa: E402
 from genesis_amd import scenes  # noqa: E402
+from genesis_amd.profiling import fused_kernel  # noqa: E402
 
 HBM_PEAK_GBPS = 8000.0
 FP32_VECTOR_PEAK_TFLOPS = 157.3  # MI355X published FP32 vector peak (counts an FMA as 2 and packed FP32)
@@ -419,7 +420,8 @@ def main():
     bytes_per_env_step = algorithmic_bytes_per_env_step(model, nb_f)
     kernel_ms = gpu_ms_f / steps  # one fused launch per substep, events on the launch stream
     achieved = bytes_per_env_step * B / (kernel_ms * 1e-3) / 1e9
-    traffic, traffic_src = measured_traffic("k_fused_wave", wl, B)
+    kernel = fused_kernel(model.n_dofs)
+    traffic, traffic_src = measured_traffic(kernel, wl, B)
     out = {
         "metric": "env-steps/s at Franka×4096 (fused vs plain GPU, FP32); p50/p99 step latency",
         "value": value,
@@ -445,7 +447,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic, "traffic_source": traffic_src,
                      "bytes_per_env_step": bytes_per_env_step, "mean_overlap_pairs": nb_f,
-                     "kernel": "k_fused_wave", "kernel_ms": kernel_ms},
+                     "kernel": kernel, "kernel_ms": kernel_ms},
         "valu_roofline": valu_roofline(wl, kernel_ms, B),
         "errno": errno,
     }

@@ -486,7 +486,7 @@ static int fused_substep(const rs_model* m, const DState& st, hipStream_t s) {
     const size_t lds = (size_t)epb * fa.lds_wave * 4;
     // one kernel variant per (private region, occupancy) for models with a row tile; models without one run the
     // generic-solver variants at the compiler's register budget (each class is instantiated in its own translation
-    // unit: rs_fused_t16.hip, rs_fused_t24.hip, rs_fused_gen.hip)
+    // unit: rs_fused_t16.hip, rs_fused_t24.hip, rs_fused_gen.hip, rs_fused_gen_lds.hip)
     const bool lds_on = m->use_lds != 0;
     if (fa.tiled == kTileMaxDofs) launch_fused_tile16(lds_on, m->occupancy, grid, block, lds, s, m->dm, st, fa);
     else if (fa.tiled == kTileWideDofs) launch_fused_tile24(lds_on, m->occupancy, grid, block, lds, s, m->dm, st, fa);
@@ -927,6 +927,7 @@ int rs_batch_create(int max_segments, rs_batch** out) {
 
 void rs_batch_destroy(rs_batch* bt) {
     if (!bt) return;
+    if (bt->side) (void)hipStreamSynchronize(bt->side);
     for (int i = 0; i < rs_batch::kRing; i++) {
         if (bt->done[i]) {
             (void)hipEventSynchronize(bt->done[i]);
@@ -935,7 +936,6 @@ void rs_batch_destroy(rs_batch* bt) {
         if (bt->dev[i]) (void)hipFree(bt->dev[i]);
         if (bt->host[i]) (void)hipHostFree(bt->host[i]);
     }
-    if (bt->side) (void)hipStreamSynchronize(bt->side);
     if (bt->side) (void)hipStreamDestroy(bt->side);
     if (bt->fork) (void)hipEventDestroy(bt->fork);
     if (bt->join) (void)hipEventDestroy(bt->join);

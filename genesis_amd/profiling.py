@@ -12,7 +12,7 @@
 * ``source_digest()``: digest of the kernel sources and build flags, recorded with a profile so that a report can tell
   whether the profile belongs to the kernels it is reporting on.
 
-Command line: ``python -m genesis_amd.profiling --trace DIR --fetch DIR --write DIR --kernel k_fused_wave
+Command line: ``python -m genesis_amd.profiling --trace DIR --fetch DIR --write DIR --kernel k_fused_
 --copy-bytes N --out profiles/NAME`` writes ``NAME.md`` (tables and figures) and ``NAME.json`` (the figures).
 """
 
@@ -27,6 +27,12 @@ import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CALIBRATION_MATCH = "elementwise"  # torch's elementwise kernel that bench.py's copy calibration launches
+ROW_TILE_MAX_DOFS = 24  # rs_wave.h kTileWideDofs
+
+
+def fused_kernel(n_dofs: int) -> str:
+    """Name of the fused substep's kernel for a model of ``n_dofs``."""
+    return "k_fused_wave" if n_dofs <= ROW_TILE_MAX_DOFS else "k_fused_large"
 
 
 def source_digest() -> str:
@@ -149,7 +155,7 @@ def main():
     ap.add_argument("--trace", required=True)
     ap.add_argument("--fetch", required=True)
     ap.add_argument("--write", required=True)
-    ap.add_argument("--kernel", default="k_fused_wave")
+    ap.add_argument("--kernel", default="k_fused_", help="part of the kernel's name (fused_kernel)")
     ap.add_argument("--copy-bytes", type=int, default=1 << 30)
     ap.add_argument("--bench-json", default=None, help="bench.py output of the traced run")
     ap.add_argument("--title", default="")

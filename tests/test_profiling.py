@@ -45,6 +45,12 @@ def test_kernel_stats_table(tmp_path):
     assert s[0]["name"] == "k_fused_wave" and s[0]["calls"] == 200 and abs(s[0]["avg_us"] - 1200.0) < 1e-9
 
 
+def test_fused_kernel_follows_the_row_tile_classes():
+    with open(os.path.join(os.path.dirname(profiling.__file__), "csrc", "rs_wave.h")) as f:
+        assert f"constexpr int kTileWideDofs = {profiling.ROW_TILE_MAX_DOFS};" in f.read()
+    assert [profiling.fused_kernel(d) for d in (9, 24, 25, 120)] == ["k_fused_wave"] * 2 + ["k_fused_large"] * 2
+
+
 def test_source_digest_is_stable():
     assert profiling.source_digest() == profiling.source_digest()
 
