@@ -957,21 +957,23 @@ int rs_batch_step(rs_batch* bt, int n, const rs_model* const* models, void* cons
     if (bt->pending[k]) HIP_OK(hipEventSynchronize(bt->done[k]));
     // Models with a row tile and larger ones want different launches: the first two environments per workgroup and their
     // private regions in LDS, the second all registers of a SIMD per wavefront. In one launch every environment takes the
-    // second's shape, which costs the first more the more of them there are; two launches side by side (they run one after
-    // the other where both streams share a hardware queue) pay off from about four environments per SIMD. 4 ticks, one
-    // launch -> two: 8 piles with 4096 quadrupeds 11.6 -> 7.5 ms, with 16384 28.0 -> 9.7; 1024 piles with 8192 quadrupeds
-    // 61.7 -> 13.9. 150 piles with 2000 small environments 8.3 -> 8.4 side by side, about 11 one after the other.
+    // second's shape, which costs the first more the more of them there are. Two launches side by side run one after the
+    // other where both streams share a hardware queue, so they are made where their sum is the shorter as well: from four
+    // environments per SIMD on, of models with mesh geoms from sixteen (those wait for the few environments with deep
+    // contacts, in either shape). 4 ticks, one launch / two / their sum: 8 piles with 4096 quadrupeds 11.6 / 7.5 / 9.4 ms,
+    // with 16384 28.0 / 9.7 / 16.4; 1024 piles with 8192 quadrupeds 61.7 / 13.9 / 15.5. 8 piles with 4096 arms 10.7 / 8.8 /
+    // 14.9, with 12288 18.2 / 13.7 / 20.0; 150 piles with 1500 quadrupeds and 500 arms 8.3 / 8.4 / 11.
     struct Launch {
         int first, n, epb, blocks, slice;
         bool use_lds;
     } launch[2];
-    int64_t n_tiled = 0;
+    int64_t n_small = 0;
     bool any_large = false;
     for (int i = 0; i < n; i++) {
-        if (models[i]->fa.tiled) n_tiled += n_envs[i];
+        if (models[i]->fa.tiled) n_small += models[i]->has_mesh ? n_envs[i] / 4 : n_envs[i];
         else any_large = true;
     }
-    const bool split = any_large && n_tiled >= (int64_t)kSplitEnvsPerCu * models[0]->n_cu;
+    const bool split = any_large && n_small >= (int64_t)kSplitEnvsPerCu * models[0]->n_cu;
     // launch[1] takes the larger models, and the others too when the launch is not split
     auto in_class = [&](int i, int large) { return (any_large && !(split && models[i]->fa.tiled)) == (large != 0); };
     FusedSegment* tab = bt->host[k];

@@ -184,14 +184,14 @@ def test_nan_velocity_spreads_as_in_the_per_stage_step(tmp_path, name, in_lds):
 def test_shared_launch_of_both_classes_equals_the_launches_alone(tmp_path, n_small):
     """Row-tile models and larger ones (region in LDS when alone, collision-free, the most dofs of the matrix-core path, and
     beyond it) in one shared step: bit for bit the steps of each alone, with only the caller's stream to wait for. With few
-    small environments the step is one launch, with 4200 it is two on two streams."""
+    small environments the step is one launch, with 4200 quadrupeds it is two on two streams."""
     from genesis_amd import runtime as rt
 
     rt.load_library()
     models = [scenes.franka_model(), _boxes(5, 0.099, OPTIONS["sat"]), _boxes(22, 0.0995, OPTIONS["sat"]),
               scenes.quadruped_model(), _loops(tmp_path, 3, OPTIONS["alone"]), _arms(tmp_path, 64, OPTIONS["alone"])]
     assert [m.n_dofs for m in models] == [9, 30, 132, 18, 30, 128]
-    sizes = [n_small, 9, 5, n_small, 7, 3]
+    sizes = [n_small, 9, 5, 2 * n_small, 7, 3]
     alone, mixed = [], []
     for m, n in zip(models, sizes):
         dm = rt.DeviceModel(m)
